@@ -220,6 +220,7 @@ struct NearIn {
     int n_tiles, n_src, n_tgt, slots, max_items, rows;
     long long max_partials;
     float kabs, q, p, log_eps;  // node count constants, ln(4 / eps)
+    float dyadic;               // rate along s of the dyadic's 1 / (k R) and 1 / (k R)^2, 0: scalar
     float small[kNearSmall];    // small[n]: largest K for which n nodes do by the small-K bound
     float pair_cycles, direct_cycles, series_cycles, fixed_cycles, sort_cycles;   // sort_cycles: 0 where no sorting pass is launched
 };
@@ -340,14 +341,18 @@ __global__ __launch_bounds__(1024) void k_near_plan(NearIn in, NearWs w) {
     const float ha = fmaxf((float)half[0], 1e-6f), hb = fmaxf((float)half[1], 1e-6f);
     const float hs = fmaxf((float)half[fit ? 3 : 2], 1e-7f * r1);
     const float grow = 1.f / (1.f - fminf(near, 0.5f));
-    // radial phase and amplitude rates per unit of s
-    const float radial = 1.1f * grow * grow * in.kabs * 0.5f * rho * rho + 2.f * rho * grow, tilt = radial * slope;
+    // radial phase and amplitude rates per unit of s: those that vanish with the
+    // sources' extent, and with the dyadic's own
+    const float smooth = 1.1f * grow * grow * in.kabs * 0.5f * rho * rho + 2.f * rho * grow;
+    const float radial = smooth + in.dyadic, tilt = radial * slope;
     const float cap = fminf(1.5f, 0.8f * acoshf(1.f / near));
     int nr = 0;
     if (on) {
         // no further than four fifths of the way to the singularity at s = 1 / rho
         const float far = 1.f + fmaxf(0.f, (0.8f / rho - r1) / hs);
-        nr = (int)fmaxf(near_count(radial * hs, in), ceilf(in.log_eps / __logf(far + sqrtf(far * far - 1.f))));
+        const float least = ceilf(in.log_eps / __logf(far + sqrtf(far * far - 1.f)));
+        // the dyadic is a polynomial of degree two in s: two more nodes always do
+        nr = (int)fminf(fmaxf(near_count(smooth * hs, in), least) + 2.f, fmaxf(near_count(radial * hs, in), least));
         if (tid < kNearMaxPatches * kNearMaxPatches) {
             const int pa = tid / kNearMaxPatches + 1, pb = tid % kNearMaxPatches + 1;
             const float na = near_axis(in, ha / pa, ex, ey, ez, tilt, la, lb, grow, cap);
@@ -698,6 +703,7 @@ int launch_near_cheb_plan(int mode, int precision, int sums, const SumPlan &p, c
         in.small[n] = 2.f * std::exp((std::lgamma(n + 1.f) + 0.693f - in.log_eps) / n);
     }
     in.small[0] = 0.f;
+    in.dyadic = mode == PYPO_MODE_SCALAR ? 0.f : (float)(1.5 / kabs);
     in.pair_cycles = (float)pair_cycles(mode, sums);
     in.direct_cycles = direct_cycles > 0.0 ? (float)direct_cycles : in.pair_cycles;
     // a coefficient's share of a target's series, and with its gradient; the passes around them
