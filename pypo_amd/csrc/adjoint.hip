@@ -67,6 +67,9 @@ __global__ __launch_bounds__(256) void k_adj_reverse32(const TgtRec32 *__restric
     const RevSplit rs = rev_split(plan, n_targets, chunk_t, gridDim.y);
     const int n_tgt = rs.n, chunk = rs.chunk;
     if ((int)blockIdx.y >= rs.used) return;
+    // A plan's few nodes carry what many targets did: their FP32 partial sums are
+    // larger against the total, so they are folded eight times as often.
+    const int step = plan && plan->on ? TILE / 8 : TILE;
     __shared__ TgtRec32 tile[TILE];
     const int tid = threadIdx.x;
     double px[SPL], py[SPL], pz[SPL];
@@ -97,39 +100,42 @@ __global__ __launch_bounds__(256) void k_adj_reverse32(const TgtRec32 *__restric
             tile[tid] = z;   // zero A: adds nothing
         }
         __syncthreads();
+#pragma unroll 1
+        for (int s0 = 0; s0 < TILE; s0 += step) {
 #pragma unroll 2
-        for (int s = 0; s < TILE; s++) {
-            const TgtRec32 &r = tile[s];
-            const float a[6] = {r.a[0], r.a[1], r.a[2], r.a[3], r.a[4], r.a[5]};
+            for (int s = s0; s < s0 + step; s++) {
+                const TgtRec32 &r = tile[s];
+                const float a[6] = {r.a[0], r.a[1], r.a[2], r.a[3], r.a[4], r.a[5]};
 #pragma unroll
-            for (int j = 0; j < SPL; j++) {
-                double rev = __builtin_fma(pz[j], r.uz, __builtin_fma(py[j], r.uy, px[j] * r.ux));
-                float f = (float)__builtin_amdgcn_fract(rev);
-                float sn, cs;
-                sincos_rev_f32(f, sn, cs);
-                float w = __builtin_fmaf(nz[j], r.rz, __builtin_fmaf(ny[j], r.ry, nx[j] * r.rx));
-                cs = (w < 0.f) ? 0.f : cs;
-                sn = (w < 0.f) ? 0.f : sn;
-                const float wc = w * cs, ws = w * sn;
-                float *c = acc[j];
+                for (int j = 0; j < SPL; j++) {
+                    double rev = __builtin_fma(pz[j], r.uz, __builtin_fma(py[j], r.uy, px[j] * r.ux));
+                    float f = (float)__builtin_amdgcn_fract(rev);
+                    float sn, cs;
+                    sincos_rev_f32(f, sn, cs);
+                    float w = __builtin_fmaf(nz[j], r.rz, __builtin_fmaf(ny[j], r.ry, nx[j] * r.rx));
+                    cs = (w < 0.f) ? 0.f : cs;
+                    sn = (w < 0.f) ? 0.f : sn;
+                    const float wc = w * cs, ws = w * sn;
+                    float *c = acc[j];
 #pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    const float ar = a[2 * q], ai = a[2 * q + 1];
-                    c[2 * q] = __builtin_fmaf(ar, cs, c[2 * q]);
-                    c[2 * q] = __builtin_fmaf(-ai, sn, c[2 * q]);
-                    c[2 * q + 1] = __builtin_fmaf(ar, sn, c[2 * q + 1]);
-                    c[2 * q + 1] = __builtin_fmaf(ai, cs, c[2 * q + 1]);
-                    c[6 + 2 * q] = __builtin_fmaf(ar, wc, c[6 + 2 * q]);
-                    c[6 + 2 * q] = __builtin_fmaf(-ai, ws, c[6 + 2 * q]);
-                    c[7 + 2 * q] = __builtin_fmaf(ar, ws, c[7 + 2 * q]);
-                    c[7 + 2 * q] = __builtin_fmaf(ai, wc, c[7 + 2 * q]);
+                    for (int q = 0; q < 3; q++) {
+                        const float ar = a[2 * q], ai = a[2 * q + 1];
+                        c[2 * q] = __builtin_fmaf(ar, cs, c[2 * q]);
+                        c[2 * q] = __builtin_fmaf(-ai, sn, c[2 * q]);
+                        c[2 * q + 1] = __builtin_fmaf(ar, sn, c[2 * q + 1]);
+                        c[2 * q + 1] = __builtin_fmaf(ai, cs, c[2 * q + 1]);
+                        c[6 + 2 * q] = __builtin_fmaf(ar, wc, c[6 + 2 * q]);
+                        c[6 + 2 * q] = __builtin_fmaf(-ai, ws, c[6 + 2 * q]);
+                        c[7 + 2 * q] = __builtin_fmaf(ar, ws, c[7 + 2 * q]);
+                        c[7 + 2 * q] = __builtin_fmaf(ai, wc, c[7 + 2 * q]);
+                    }
                 }
             }
+#pragma unroll
+            for (int j = 0; j < SPL; j++)
+#pragma unroll
+                for (int q = 0; q < 12; q++) { tot[j][q] += (double)acc[j][q]; acc[j][q] = 0.f; }
         }
-#pragma unroll
-        for (int j = 0; j < SPL; j++)
-#pragma unroll
-            for (int q = 0; q < 12; q++) { tot[j][q] += (double)acc[j][q]; acc[j][q] = 0.f; }
     }
 #pragma unroll
     for (int j = 0; j < SPL; j++) {

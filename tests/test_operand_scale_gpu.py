@@ -34,13 +34,15 @@ def test_small_sources_beside_one_in_shadow(hip, n_src, ratio):
     assert err <= 1e-6
 
 
-def test_gradient_of_a_beam_is_as_good_as_its_sums(hip):
+@pytest.mark.parametrize("kernel,bar", [("matrix", 1.9e-7), ("vector", 2.1e-7)])
+def test_gradient_of_a_beam_is_as_good_as_its_sums(hip, kernel, bar):
     """Gradient of a far-field fit, mixed against FP64 for the same far field.
     Summed over every far-field target it is off by 1.7e-7 to 2.4e-7 of its norm
-    (FP32 currents and phases; rms of these four 1.9e-7); the sums at Chebyshev
-    nodes have to be no worse."""
+    (FP32 currents and phases; rms of these four 1.9e-7, 2.1e-7 on the vector
+    ALUs); the sums at Chebyshev nodes have to be no worse."""
     import torch
     from pypo_amd import adjoint as PA
+    from pypo_amd import bind as B
     feed, cur, dish, ff, k, radius = PA.surface_error_workload(n_dish=401, n_ff=151, n_feed=33)
     prob = PA.ShapeProblem(feed, cur, dish, ff, k)
     x, y = prob.g_dish0[0].cpu().numpy(), prob.g_dish0[1].cpu().numpy()
@@ -50,7 +52,11 @@ def test_gradient_of_a_beam_is_as_good_as_its_sums(hip):
         d = torch.tensor(PA.zernike_displacement(x, y, radius, sigma=0.02, seed=seed), device="cuda")
         e = prob.far_field(d, "fp64")
         g = 2 * ((e[0:6] ** 2).sum(0) - ideal) / ideal.max() ** 2
-        ref, got = (prob.power_grad(d, e, g, p) for p in ("fp64", "mixed"))
+        B.set_ff_kernel(kernel)
+        try:
+            ref, got = (prob.power_grad(d, e, g, p) for p in ("fp64", "mixed"))
+        finally:
+            B.set_ff_kernel("matrix")
         errs.append((torch.linalg.norm(got - ref) / torch.linalg.norm(ref)).item())
-    print("gradient errors", ["%.2e" % v for v in errs])
-    assert np.sqrt(np.mean(np.square(errs))) <= 1.9e-7
+    print(kernel, "gradient errors", ["%.2e" % v for v in errs])
+    assert np.sqrt(np.mean(np.square(errs))) <= bar
