@@ -200,9 +200,10 @@ __global__ __launch_bounds__(1024) void k_cheb_plan(PlanIn in, ChebWs w) {
         for (int i = tid; i < pl.n; i += 1024) cheb_node(pl, i, w.th, w.ph);
 }
 
+template <bool TURNED>
 __global__ __launch_bounds__(256) void k_cheb_reduce(const double *__restrict__ partial, ChebWs w, double rev_scale) {
     if (!w.plan->on) return;
-    cheb_reduce(w, partial, rev_scale, blockIdx.x, gridDim.x);
+    cheb_reduce<TURNED>(w, partial, rev_scale, blockIdx.x, gridDim.x);
     cheb_check_rows(w, blockIdx.x, gridDim.x);
 }
 
@@ -281,8 +282,9 @@ int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int 
     return 0;
 }
 
-int launch_cheb_coef(const double *partial, const ChebWs &w, double rev_scale, hipStream_t st) {
-    hipLaunchKernelGGL(k_cheb_reduce, dim3(512), dim3(256), 0, st, partial, w, rev_scale);
+int launch_cheb_coef(int precision, const double *partial, const ChebWs &w, double rev_scale, hipStream_t st) {
+    hipLaunchKernelGGL(precision == PYPO_PREC_FP64 ? k_cheb_reduce<true> : k_cheb_reduce<false>, dim3(512), dim3(256), 0,
+                       st, partial, w, rev_scale);
     PYPO_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_cheb_coef, dim3(1024), dim3(256), 0, st, w);
     PYPO_CHECK_LAUNCH();

@@ -250,7 +250,7 @@ double far_cycles(int precision);
 int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int n_src, double rev_scale,
                      size_t partial_bytes, double cycles, double fixed_us, double extra, const ChebWs &w,
                      hipStream_t st);
-int launch_cheb_coef(const double *partial, const ChebWs &w, double rev_scale, hipStream_t st);
+int launch_cheb_coef(int precision, const double *partial, const ChebWs &w, double rev_scale, hipStream_t st);
 // Workgroups of 256 lanes one CU holds at once for the far-field sum kernel
 // that launch_ff_sum / launch_ff_mfma pick for (precision, targets per lane).
 int ff_wgs_per_cu(int precision, int tpl);

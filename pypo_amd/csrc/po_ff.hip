@@ -263,6 +263,12 @@ __device__ __forceinline__ void ff_tile_fp64(const SrcRec64 *tile, const double 
     }
 }
 
+// At the nodes of a plan that is on, phases are formed from cos(theta) - 1 and
+// the sources carry exp(j 2 pi (z - c_z) rev_scale): cos(theta) itself rounds
+// to 2^-54, which times z is common to all sources of a node and would come
+// back in every target (300 wavelengths of dish, 2500 from the origin: error
+// 4.7e-14 with cos(theta), 1.6e-15 like this).  cheb_reduce takes the same part
+// out again.  One sincos a record and workgroup, of 512 pairs.
 template <int TPL, bool PART>
 __global__ __launch_bounds__(256) void k_ff_fp64(const SrcRec64 *__restrict__ src,
                                                  const TileMeta *__restrict__ meta, int n_src,
@@ -277,6 +283,7 @@ __global__ __launch_bounds__(256) void k_ff_fp64(const SrcRec64 *__restrict__ sr
     const double *th = ft.th, *ph = ft.ph;
     const int tb = ft.tb, sp = ft.sp, n_tgt = ft.n;
     chunk = ft.chunk;
+    const bool nodes = w.plan && w.plan->on;
     double ux[TPL], uy[TPL], uz[TPL];
     double rx[TPL], ry[TPL], rz[TPL];
     Cone cone;
@@ -285,16 +292,17 @@ __global__ __launch_bounds__(256) void k_ff_fp64(const SrcRec64 *__restrict__ sr
 #pragma unroll
         for (int j = 0; j < TPL; j++) {
             int t = tb * (TILE * TPL) + j * TILE + tid;
-            double x = 0, y = 0, z = 0;
+            double x = 0, y = 0, z = 0, v = 0;
             if (t < n_tgt) {
                 double st, ct, sp, cp;
                 sincos(th[t], &st, &ct);
                 sincos(ph[t], &sp, &cp);
                 x = cp * st; y = sp * st; z = ct;
+                v = nodes ? cos_less_one(th[t]) : z;
             }
             if (j == 0) any = t < n_tgt;
             ux[j] = x; uy[j] = y; uz[j] = z;
-            rx[j] = x * rev_scale; ry[j] = y * rev_scale; rz[j] = z * rev_scale;
+            rx[j] = x * rev_scale; ry[j] = y * rev_scale; rz[j] = v * rev_scale;
         }
         cone = block_cone((float)ux[0], (float)uy[0], (float)uz[0], any, scratch);
         if (TPL > 1 && cone.cos_half > 0.f) {
@@ -321,6 +329,16 @@ __global__ __launch_bounds__(256) void k_ff_fp64(const SrcRec64 *__restrict__ sr
     for (int base = s_begin; base < s_end; base += TILE) {
         __syncthreads();
         ld.store(reinterpret_cast<uint4 *>(tile), tid);
+        if (nodes) {   // each lane its own record
+            double sn, cs;
+            sincos_rev_f64(__builtin_amdgcn_fract((tile[tid].z - w.plan->c[2]) * rev_scale), sn, cs);
+#pragma unroll
+            for (int q = 0; q < 12; q += 2) {
+                const double re = tile[tid].c[q], im = tile[tid].c[q + 1];
+                tile[tid].c[q] = re * cs - im * sn;
+                tile[tid].c[q + 1] = re * sn + im * cs;
+            }
+        }
         __syncthreads();
         if (base + TILE < s_end) ld.load(g, base + TILE + tid, s_end);
         const TileMeta m = meta[base / TILE];

@@ -168,7 +168,7 @@ int launch_po(const SumPlan &p, int mode, int precision, const void *packed, int
     if (err) return err;
     tm.stop();
 
-    if (cw.plan && (err = launch_cheb_coef(partial_ws, cw, rev_scale, st))) return err;
+    if (cw.plan && (err = launch_cheb_coef(precision, partial_ws, cw, rev_scale, st))) return err;
     if (nw.plan && (err = launch_near_cheb_coef(mode, partial_ws, nw, carrier, st))) return err;
     if (mode == PYPO_MODE_FF)
         return launch_ff_finish(p, ct, n_tgt, rev_scale, t_dir, pc.prefactor, *(const c2Bundle *)res, partial_ws, cw,

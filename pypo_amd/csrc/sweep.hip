@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void k_sweep_cheb_nodes(const ChebWs *__restri
 __global__ __launch_bounds__(256) void k_sweep_cheb_reduce(const StageInst *__restrict__ insts,
                                                            const ChebWs *__restrict__ ws) {
     const ChebWs w = ws[blockIdx.y];
-    if (w.plan) cheb_reduce(w, insts[blockIdx.y].partial, insts[blockIdx.y].rev_scale, blockIdx.x, gridDim.x);
+    if (w.plan) cheb_reduce<false>(w, insts[blockIdx.y].partial, insts[blockIdx.y].rev_scale, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_sweep_cheb_coef(const ChebWs *__restrict__ ws) {
