@@ -544,6 +544,15 @@ void callRTKernel(reflparamsf ctp, cframef *fr_in, cframef *fr_out, float epsilo
 int pypo_hip_set_timing(int enable);
 double pypo_hip_last_kernel_ms(void);
 
+/* What the last pypo_hip_propagate_dev, drop-in propagation or
+ * pypo_hip_ff_power_grad_dev call with timing enabled did about Chebyshev
+ * grids: info[0..3] of a far field's directions { 0 not tried / 1 tried and
+ * off / 2 on, nodes, nodes along the first axis, targets a row or 0 }, info[4..7]
+ * of a near field's patches { the same, nodes, patches, nodes along 1 / R }.
+ * Diagnostic: such a call waits for its kernels.  Zeros if unavailable (no such
+ * call yet, or it was captured into a graph). */
+int pypo_hip_last_grids(int info[8]);
+
 #ifdef __cplusplus
 }
 #endif

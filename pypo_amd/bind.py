@@ -91,6 +91,8 @@ def loadHIPlib():
         lib.pypo_hip_set_timing.restype = i
         lib.pypo_hip_last_kernel_ms.argtypes = []
         lib.pypo_hip_last_kernel_ms.restype = d
+        lib.pypo_hip_last_grids.argtypes = [P(i)]
+        lib.pypo_hip_last_grids.restype = i
         lib.pypo_hip_propagate_dev.argtypes = [i, ctypes.c_void_p, P(PS.reflcontainer),
                                                P(PS.reflcontainer), ctypes.c_void_p, i, i, i, d, d, d,
                                                i, ctypes.c_void_p]

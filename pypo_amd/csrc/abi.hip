@@ -68,6 +68,7 @@ int g_precision = PYPO_PREC_MIXED;
 int g_rt_max_iter = 50;
 bool g_timing = false;
 double g_last_ms = -1.0;
+int g_last_grids[8] = {};
 
 int ensure_init() {
     if (g_stream) return 0;
@@ -123,6 +124,7 @@ int end_call(hipStream_t st) {
 }  // namespace
 
 void record_kernel_ms(double ms) { g_last_ms = ms; }
+void record_grids(const int (&info)[8]) { std::copy(info, info + 8, g_last_grids); }
 
 hipStream_t lib_stream(int *err) {
     *err = ensure_init();
@@ -588,6 +590,13 @@ int pypo_hip_set_timing(int enable) {
 }
 
 double pypo_hip_last_kernel_ms(void) { return g_last_ms; }
+
+int pypo_hip_last_grids(int info[8]) {
+    std::lock_guard<std::recursive_mutex> lock(g_mu);
+    PYPO_REQUIRE(info, ERR_ARG, "last_grids: NULL argument");
+    std::copy(g_last_grids, g_last_grids + 8, info);
+    return 0;
+}
 
 // ---- drop-in PO entry points (InterfaceCPU.h:24-58) ---------------------------
 
@@ -1358,7 +1367,7 @@ int pypo_hip_ff_power_grad_dev(const reflcontainer *dish, int gmode, int ncx, in
                                     grid_ptrs(*feed), feed->size, feed_gmode,
                                     feed_ncx, feed_ncy, bundle12(*feed_currents), grid_ptrs(*ff),
                                     ff->size, bundle12(*ff_fields), dl_dp, k, t_direction, grad, ws,
-                                    wsb, st)))
+                                    wsb, st, g_timing)))
         return err;
     return end_call(st);
 }

@@ -888,7 +888,7 @@ int launch_ff_power_grad(int precision, const GridPtrs &dish, int n_dish, int gm
                          const GridPtrs &feed, int n_feed, int fgmode, int fncx,
                          int fncy, const Bundle12 &feed_cur, const GridPtrs &ff, int n_tgt,
                          const Bundle12 &E, const double *g, double k, double tdir, double *grad,
-                         void *ws, size_t ws_bytes, hipStream_t st) {
+                         void *ws, size_t ws_bytes, hipStream_t st, bool time_it) {
     PYPO_REQUIRE(n_dish > 0 && n_feed > 0 && n_tgt > 0, ERR_ARG, "adjoint: empty grid");
     PYPO_REQUIRE((long long)ncx * ncy == n_dish && (long long)fncx * fncy == n_feed, ERR_ARG,
                  "adjoint: n_cells do not match the grid sizes");
@@ -959,7 +959,7 @@ int launch_ff_power_grad(int precision, const GridPtrs &dish, int n_dish, int gm
         hipLaunchKernelGGL(k_adj_combine, dim3(blocks), dim3(256), 0, st, part, splits, dish, n_dish, gmode,
                            ncx, ncy, jd, p.fsplits, k, tdir, grad, far.w.plan, near.plan);
     PYPO_CHECK_LAUNCH();
-    return 0;
+    return time_it ? read_plans(far.w, near, st) : 0;
 }
 
 }  // namespace pypo

@@ -290,7 +290,7 @@ int launch_ff_power_grad(int precision, const GridPtrs &dish, int n_dish, int gm
                          const GridPtrs &feed, int n_feed, int fgmode, int fncx,
                          int fncy, const Bundle12 &feed_cur, const GridPtrs &ff, int n_tgt,
                          const Bundle12 &E, const double *g, double k, double tdir, double *grad,
-                         void *ws, size_t ws_bytes, hipStream_t st);
+                         void *ws, size_t ws_bytes, hipStream_t st, bool time_it);
 
 // Beam initialisation (beam.hip).  Grids and bundles are device memory.
 int launch_gauss(const GPODict &g, const GridPtrs &gr, int n, const Bundle12 &field, const Bundle12 &cur,
@@ -330,5 +330,6 @@ int launch_frame_stats(const FrameView &f, int n, double *ws, double *out8, hipS
 
 // Kernel timing of the last timed launch (HIP events on the launch stream).
 void record_kernel_ms(double ms);
+void record_grids(const int (&info)[8]);
 
 }  // namespace pypo

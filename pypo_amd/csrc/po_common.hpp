@@ -276,6 +276,8 @@ int near_wgs_per_cu(int mode, int precision);
 // pairs of what the plan would save, 0: the mode's own sum.
 int launch_near_cheb_plan(int mode, int precision, int sums, const SumPlan &p, const TileMeta *meta, int n_src, double kabs,
                           size_t partial_bytes, double direct_cycles, const NearWs &w, hipStream_t st);
+// Plans of the call on st for pypo_hip_last_grids; waits for them.
+int read_plans(const ChebWs &far, const NearWs &near, hipStream_t st);
 int launch_near_cheb_coef(int mode, const double *partial, const NearWs &w, double rev_scale, hipStream_t st);
 int launch_scalar_sum(int precision, const SumPlan &p, const void *packed, int n_src,
                       const GridPtrs &ct, int n_tgt, double rev_scale, double *partial, const NearWs &w,

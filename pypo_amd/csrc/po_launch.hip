@@ -131,6 +131,32 @@ SumPlan plan_cap_splits(const SumPlan &p, int n_src, int max_splits) {
     return q;
 }
 
+int read_plans(const ChebWs &far, const NearWs &near, hipStream_t st) {
+    int info[8] = {};
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        ChebPlan f;
+        NearPlan n;
+        int not_rows = 0;
+        if (far.plan) {
+            PYPO_HIP_TRY(hipMemcpyAsync(&f, far.plan, sizeof(f), hipMemcpyDeviceToHost, st));
+            PYPO_HIP_TRY(hipMemcpyAsync(&not_rows, far.not_rows, sizeof(int), hipMemcpyDeviceToHost, st));
+        }
+        if (near.plan) PYPO_HIP_TRY(hipMemcpyAsync(&n, near.plan, sizeof(n), hipMemcpyDeviceToHost, st));
+        PYPO_HIP_TRY(hipStreamSynchronize(st));
+        if (far.plan) {
+            info[0] = f.on ? 2 : 1;
+            if (f.on) { info[1] = f.n; info[2] = f.na; info[3] = not_rows ? 0 : f.row; }
+        }
+        if (near.plan) {
+            info[4] = n.on ? 2 : 1;
+            if (n.on) { info[5] = n.n; info[6] = n.pa * n.pb; info[7] = n.nr; }
+        }
+    }
+    record_grids(info);
+    return 0;
+}
+
 int launch_po(const SumPlan &p, int mode, int precision, const void *packed, int n_src, const GridPtrs &ct,
               int n_tgt, double k, double epsilon, double t_dir, void *res, double *partial_ws, size_t ws_bytes,
               const ChebWs *cheb, const NearWs *near, hipStream_t st, bool time_it) {
@@ -170,6 +196,7 @@ int launch_po(const SumPlan &p, int mode, int precision, const void *packed, int
 
     if (cw.plan && (err = launch_cheb_coef(precision, partial_ws, cw, rev_scale, st))) return err;
     if (nw.plan && (err = launch_near_cheb_coef(mode, partial_ws, nw, carrier, st))) return err;
+    if (time_it && (err = read_plans(cw, nw, st))) return err;
     if (mode == PYPO_MODE_FF)
         return launch_ff_finish(p, ct, n_tgt, rev_scale, t_dir, pc.prefactor, *(const c2Bundle *)res, partial_ws, cw,
                                 st);
