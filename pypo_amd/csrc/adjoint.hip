@@ -290,22 +290,29 @@ __device__ __forceinline__ void rev_tile_mfma(const RevTile &tt, const mfma::hal
 // Partial layout [split][24][n_src]: q 0..5 = B, 6..11 = G_x, 12..17 = G_y,
 // 18..23 = G_z (re/im xyz interleaved).  Grid: (dish blocks of 64 MB points,
 // target splits).
+// NODES: the targets are a plan's few nodes, which carry what many targets did:
+// their FP32 partial sums are larger against the total, and are folded four
+// times as often.  A form of its own: with the fold's distance as a variable the
+// sums over all targets lost 7 to 19 % where a launch leaves CUs idle.
 template <int MB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_reverse_mfma(
-    const TgtRec32 *__restrict__ tg, const TileMeta *__restrict__ tmeta, int n_targets, int chunk_t, GridPtrs src,
-    int n_src, double *__restrict__ partial, const ChebPlan *plan) {
-    const RevSplit rs = rev_split(plan, n_targets, chunk_t, gridDim.y);
-    const int n_tgt = rs.n, chunk = rs.chunk;
-    if ((int)blockIdx.y >= rs.used) return;
-    // A plan's few nodes carry what many targets did: their FP32 partial sums
-    // are larger against the total, so they are folded four times as often.
-    const int step = plan && plan->on ? mfma::KSTEPS / 4 : mfma::KSTEPS;
+struct RevShared {
+    RevTile tt;
+    mfma::half8 b0h[mfma::KSTEPS][64], b0l[mfma::KSTEPS][64], b1h[mfma::KSTEPS][64], b1l[mfma::KSTEPS][64];
+    float nv[3][64 * MB];   // normals of the workgroup's dish points (shadow test)
+    float scratch[4];
+};
+
+template <int MB, bool NODES>
+__device__ __forceinline__ void adj_reverse_mfma(RevShared<MB> &sh, const TgtRec32 *__restrict__ tg,
+                                                 const TileMeta *__restrict__ tmeta, int n_tgt, int chunk,
+                                                 const GridPtrs &src, int n_src, double *__restrict__ partial) {
+    constexpr int step = NODES ? mfma::KSTEPS / 4 : mfma::KSTEPS;
     using mfma::floatx4;
     using mfma::half8;
-    __shared__ RevTile tt;
-    __shared__ half8 b0h[mfma::KSTEPS][64], b0l[mfma::KSTEPS][64], b1h[mfma::KSTEPS][64], b1l[mfma::KSTEPS][64];
-    __shared__ float nv[3][64 * MB];   // normals of the workgroup's dish points (shadow test)
-    __shared__ float scratch[4];
+    RevTile &tt = sh.tt;
+    auto &b0h = sh.b0h, &b0l = sh.b0l, &b1h = sh.b1h, &b1l = sh.b1l;
+    auto &nv = sh.nv;
+    auto &scratch = sh.scratch;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int row = lane & 15, kb = lane >> 4;
     const int s0 = blockIdx.x * (64 * MB) + wave * (16 * MB);
@@ -426,6 +433,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                 }
             }
     }
+}
+
+template <int MB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_reverse_mfma(
+    const TgtRec32 *__restrict__ tg, const TileMeta *__restrict__ tmeta, int n_targets, int chunk, GridPtrs src,
+    int n_src, double *__restrict__ partial, const ChebPlan *plan) {
+    __shared__ RevShared<MB> sh;
+    const RevSplit rs = rev_split(plan, n_targets, chunk, gridDim.y);
+    if ((int)blockIdx.y >= rs.used) return;
+    if (plan && plan->on) adj_reverse_mfma<MB, true>(sh, tg, tmeta, rs.n, rs.chunk, src, n_src, partial);
+    else adj_reverse_mfma<MB, false>(sh, tg, tmeta, rs.n, rs.chunk, src, n_src, partial);
 }
 
 __global__ __launch_bounds__(256) void k_adj_reverse64(const TgtRec64 *__restrict__ tg, int n_targets,
