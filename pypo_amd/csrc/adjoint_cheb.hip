@@ -33,7 +33,12 @@ namespace pypo {
 namespace {
 
 constexpr int kMomSplits = 64;     // target splits of the moments
-constexpr int kMomA = 64, kMomB = 16, kMomT = 32;   // moments per workgroup, targets per stage
+constexpr int kMomT = 32;          // and targets per stage
+// SIMD cycles a target takes for up to kMomTiles tiles of moments: 5.8 to 6.2 ns
+// measured from 40 000 to 160 000 targets, 10 to 16 tiles.  A reverse sum over a
+// 90^2 dish and 300^2 targets at 99 x 99 nodes, 521 us of moments, is slower than
+// one over the targets (865 us of gradient against 702): the rule leaves it off.
+constexpr double kMomCycles = 6.0e-9 * kSimdHz;
 
 // Normal cone and position box per 256 dish points, then the targets' boxes.
 __global__ __launch_bounds__(256) void k_adj_dish_meta(GridPtrs dish, int n, TileMeta *__restrict__ meta, ChebWs w) {
@@ -289,11 +294,11 @@ int launch_adj_far(int precision, const AdjFar &f, const GridPtrs &dish, int n_d
     // the nodes here: the plan's own splits are not used.
     const SumPlan p{1, (w.n_tgt + TILE - 1) / TILE, n_tiles(n_dish), TILE};
     int err = launch_cheb_plan(PYPO_PREC_FP64, p, f.meta, n_dish, rev_scale, partial_bytes(PYPO_MODE_FF, p, w.n_tgt),
-                               reverse_cycles(precision), 60.0, 1.0, w, st);
+                               {reverse_cycles(precision), 60.0, 1.0, kMomCycles}, w, st);
     if (err) return err;
     hipLaunchKernelGGL(k_adj_amplitudes, dim3((w.n_tgt + 255) / 256), dim3(256), 0, st, w, E, g, rev_scale, pref, f.amp);
     PYPO_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_adj_moments, dim3(16, kMomSplits), dim3(256), 0, st, w, (const double *)f.amp, f.moments);
+    hipLaunchKernelGGL(k_adj_moments, dim3(kMomTiles, kMomSplits), dim3(256), 0, st, w, (const double *)f.amp, f.moments);
     PYPO_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_adj_moment_sum, dim3(256), dim3(256), 0, st, w, f.moments);
     PYPO_CHECK_LAUNCH();

@@ -34,8 +34,8 @@ __device__ int cheb_nodes(float kabs, float h, float x, float y, float z, float 
 // pair of the sum).  eval: the series at one target in such units -- 13 (7
 // without magnetic currents) FP64 FMAs of 4.8 issue cycles per 64 targets and
 // term, against 59 cycles per 64 pairs of the matrix kernel, 80 of the vector
-// kernel, 225 of the FP64 kernel (far_cycles; all measured on gfx950); fixed:
-// the passes between.
+// kernel, 225 of the FP64 kernel (far_cycles; all measured on gfx950), or the
+// adjoint's moments; fixed: the passes between.
 __device__ bool cheb_pays(long long n, double eval, double n_src, double n_tgt, double lanes, double fixed) {
     const double nodes = ceil((double)n / lanes) * lanes, tgts = ceil(n_tgt / lanes) * lanes;
     return nodes * n_src + eval * n_tgt + fixed < 0.8 * tgts * n_src;
@@ -46,7 +46,7 @@ struct PlanIn {
     int n_tiles;
     int n_src, n_tgt, tpl, slots, max_items;   // max_items: workgroups launched for the sum
     long long max_partials;                    // doubles of the split partials
-    double kabs, q, p, cycles, fixed, extra;
+    double kabs, q, p, cycles, fixed, extra, moments;
 };
 
 // One workgroup: reduce the extents, decide, write the plan and (w.th not null)
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(1024) void k_cheb_plan(PlanIn in, ChebWs w) {
     // grid bring a and b back to a few ulp.  One LDS atomic per wave: a
     // thousand on one word would take microseconds.
     const double tol = 2e-15 * (fabs(pl.a_mid) + pl.a_half + fabs(pl.b_mid) + pl.b_half);
-    if (pl.on && !flags[0]) {
+    if (pl.on && !flags[0] && in.moments == 0.0) {
         double a0, x;
         target_ab(w.tgt_th, w.tgt_ph, 0, a0, x);
         int first = 1 << 30;
@@ -164,9 +164,11 @@ __global__ __launch_bounds__(1024) void k_cheb_plan(PlanIn in, ChebWs w) {
         pl.row = row >= 16 && row <= kChebMaxRow && in.n_tgt % row == 0 &&
                          pl.na * row <= min(kChebMaxRows, in.n_tgt) ? row : 0;
         const double terms = pl.row ? pl.na : pl.n;
+        const int tiles = ((pl.na + kMomA - 1) / kMomA) * ((pl.nb + kMomB - 1) / kMomB);
+        const double eval = in.moments > 0.0 ? (tiles + kMomTiles - 1) / kMomTiles * in.moments * 64.0
+                                             : terms * (flags[1] ? 13.0 : 7.0) * 4.8;
         pl.on = pl.on && !flags[0] &&
-                cheb_pays(pl.n, terms * (flags[1] ? 13.0 : 7.0) * 4.8 / in.cycles, in.n_src, in.n_tgt, 256.0 * in.tpl,
-                          in.fixed);
+                cheb_pays(pl.n, eval / in.cycles, in.n_src, in.n_tgt, 256.0 * in.tpl, in.fixed);
         pl.tblocks = (pl.n + 256 * in.tpl - 1) / (256 * in.tpl);
     }
     __syncthreads();
@@ -261,8 +263,7 @@ ChebWs cheb_carve(void *base, int n_src, const GridPtrs &ct, int n_tgt) {
 }
 
 int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int n_src, double rev_scale,
-                     size_t partial_bytes, double cycles, double fixed_us, double extra, const ChebWs &w,
-                     hipStream_t st) {
+                     size_t partial_bytes, const ChebCost &cost, const ChebWs &w, hipStream_t st) {
     const bool f64 = precision == PYPO_PREC_FP64;
     PlanIn in;
     in.meta = meta;
@@ -274,9 +275,10 @@ int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int 
     in.kabs = std::fabs(rev_scale) * kTwoPi;
     in.q = f64 ? 8.9 : 6.9;
     in.p = f64 ? 10.05 : 3.05;
-    in.cycles = cycles;
-    in.fixed = fixed_us * 64.0 * kSimdHz * 1e-6 / cycles;
-    in.extra = extra;
+    in.cycles = cost.cycles;
+    in.fixed = cost.fixed_us * 64.0 * kSimdHz * 1e-6 / cost.cycles;
+    in.extra = cost.extra;
+    in.moments = cost.moments;
     hipLaunchKernelGGL(k_cheb_plan, dim3(1), dim3(1024), 0, st, in, w);
     PYPO_CHECK_LAUNCH();
     return 0;

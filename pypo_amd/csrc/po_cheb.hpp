@@ -56,6 +56,9 @@ constexpr int kChebMaxNodes = 32768;    // na nb, also the workspace's size
 constexpr int kChebMaxAxis = 224;       // na, nb
 constexpr int kChebMaxRow = 2048;       // targets per row, and na times that, of the row form
 constexpr int kChebMaxRows = 65536;
+// The adjoint's moments of the targets (adjoint_cheb.hip): tiles of kMomA x kMomB
+// moments, kMomTiles of them at a time.
+constexpr int kMomA = 64, kMomB = 16, kMomTiles = 16;
 constexpr int kChebBoxTargets = 1024;   // targets per workgroup that reduces their box
 
 struct ChebPlan {

@@ -242,14 +242,18 @@ int launch_ff_sum(int precision, const SumPlan &p, const void *packed, int n_src
                   int n_tgt, double rev_scale, double *partial, const ChebWs &w, hipStream_t st);
 int launch_ff_mfma(const SumPlan &p, const void *packed, int n_src, const GridPtrs &ct, int n_tgt,
                    double rev_scale, double *partial, const ChebWs &w, hipStream_t st);
-// Plan and nodes of the Chebyshev grid (before the sum; for the cost rule the
-// issue cycles of 64 pairs and the time of the passes it adds; extra: rate of a
-// factor beside the phase), and the coefficients of the node sums (after it).
+// Plan and nodes of the Chebyshev grid (before the sum), and the coefficients
+// of the node sums (after it).
 constexpr double kSimdHz = 1024 * 2.4e9;   // SIMD cycles per second of the chip
 double far_cycles(int precision);
+struct ChebCost {          // for the cost rule
+    double cycles;         // issue cycles of 64 pairs
+    double fixed_us;       // the passes it adds
+    double extra;          // rate of a factor beside the phase
+    double moments;        // 0: the series at the targets; else their moments' cycles per target and kMomTiles tiles
+};
 int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int n_src, double rev_scale,
-                     size_t partial_bytes, double cycles, double fixed_us, double extra, const ChebWs &w,
-                     hipStream_t st);
+                     size_t partial_bytes, const ChebCost &cost, const ChebWs &w, hipStream_t st);
 int launch_cheb_coef(int precision, const double *partial, const ChebWs &w, double rev_scale, hipStream_t st);
 // Workgroups of 256 lanes one CU holds at once for the far-field sum kernel
 // that launch_ff_sum / launch_ff_mfma pick for (precision, targets per lane).

@@ -178,8 +178,8 @@ int launch_po(const SumPlan &p, int mode, int precision, const void *packed, int
     const TileMeta *meta = (const TileMeta *)((const char *)packed + meta_offset(rb, n_src));
     int err;
 
-    if (cw.plan && (err = launch_cheb_plan(precision, p, meta, n_src, rev_scale, ws_bytes, far_cycles(precision), 30.0,
-                                           0.0, cw, st)))
+    if (cw.plan && (err = launch_cheb_plan(precision, p, meta, n_src, rev_scale, ws_bytes,
+                                           {far_cycles(precision), 30.0, 0.0, 0.0}, cw, st)))
         return err;
     if (nw.plan &&
         (err = launch_near_cheb_plan(mode, precision, precision, p, meta, n_src, std::fabs(k), ws_bytes, 0.0, nw, st)))

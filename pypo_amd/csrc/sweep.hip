@@ -530,7 +530,7 @@ int sweep_cheb(Sweep *s, const GridPtrs &gff, hipStream_t st) {
             return err;
         const SumPlan sp{2, (s->n_ff + 511) / 512, n_tiles(p.n), TILE};
         if ((err = launch_cheb_plan(PYPO_PREC_MIXED, sp, p.meta, p.n, s->ff[i].rev_scale,
-                                    partial_bytes(PYPO_MODE_FF, sp, s->n_ff), far_cycles(PYPO_PREC_MIXED), 4.0, 0.0, w, st)))
+                                    partial_bytes(PYPO_MODE_FF, sp, s->n_ff), {far_cycles(PYPO_PREC_MIXED), 4.0, 0.0, 0.0}, w, st)))
             return err;
     }
     PYPO_HIP_TRY(hipMemcpyAsync(s->cheb.data(), s->d_plans, s->n_inst * sizeof(ChebPlan), hipMemcpyDeviceToHost, st));

@@ -225,3 +225,17 @@ def test_gradient_plans(grids, port, n_dish, n_ff, n_feed, focal, ff_deg, far, n
         print(f"{n_dish}^2 x {n_ff}^2, feed {n_feed}^2, +-{ff_deg} deg {prec}: {info} {worst:.2e}")
         assert info[0] == far and info[4] == state
         assert worst <= bar
+
+
+@pytest.mark.parametrize("n_dish,n_ff,ff_deg,far", [(90, 300, 9.0, OFF), (64, 400, 6.0, OFF), (401, 121, 1.0, ON)])
+def test_gradient_plan_counts_the_moments(grids, n_dish, n_ff, ff_deg, far):
+    """A small dish under many targets: the targets' moments, one for every node
+    and target, cost more than the reverse sums they would save."""
+    import torch
+    feed, cur, dish, ff, k, _ = PA.surface_error_workload(n_dish=n_dish, n_ff=n_ff, n_feed=9, ff_deg=ff_deg,
+                                                          diameter=300.0, focal=120.0, lam=3.0)
+    prob = PA.ShapeProblem(feed, cur, dish, ff, k)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    E = torch.randn((12, n_ff * n_ff), dtype=torch.float64, device="cuda", generator=gen)
+    prob.power_grad(torch.zeros(n_dish * n_dish, dtype=torch.float64, device="cuda"), E, E[0])
+    assert grids()[0] == far
