@@ -289,21 +289,18 @@ size_t po_extra_bytes(int mode, int precision, int n_src, int n_tgt) {
     return near_cheb_try(mode, precision, n_src, n_tgt) ? near_cheb_bytes(mode, n_src, n_tgt) : 0;
 }
 
-// src: the scalar field's parts, or nullptr
-void po_extra(void *base, int mode, const GridPtrs &cs, int n_src, const GridPtrs &ct, int n_tgt, const double *u,
-              const double *v, PoWs &w) {
+void po_extra(void *base, int mode, int n_src, const GridPtrs &ct, int n_tgt, PoWs &w) {
     if (mode == PYPO_MODE_FF) w.cheb = cheb_carve(base, n_src, ct, n_tgt);
-    else w.near = near_cheb_carve(base, mode, cs, n_src, ct, n_tgt, u, v);
+    else w.near = near_cheb_carve(base, mode, n_src, ct, n_tgt);
 }
 
-int po_workspace(int mode, int precision, const GridPtrs &cs, int n_src, const GridPtrs &ct, int n_tgt,
-                 const double *u, const double *v, PoWs &w) {
+int po_workspace(int mode, int precision, int n_src, const GridPtrs &ct, int n_tgt, PoWs &w) {
     int err = 0;
     w.plan = plan_sum(mode, precision, n_src, n_tgt);
     w.bytes = (partial_bytes(mode, w.plan, n_tgt) + 255) / 256 * 256;
     const size_t extra = po_extra_bytes(mode, precision, n_src, n_tgt);
     w.partial = (double *)pool_get(SLOT_PARTIAL, w.bytes + extra, &err);
-    if (!err && extra) po_extra((char *)w.partial + w.bytes, mode, cs, n_src, ct, n_tgt, u, v, w);
+    if (!err && extra) po_extra((char *)w.partial + w.bytes, mode, n_src, ct, n_tgt, w);
     return err;
 }
 
@@ -351,16 +348,15 @@ int po_dropin(int mode, void *res, const reflparams &sp, const reflparams &tp, r
     void *packed = pool_get(SLOT_PACKED, packed_bytes(mode, prec, gs), &err);
     if (err) return err;
     PoWs ws;
-    const bool scalar = mode == PYPO_MODE_SCALAR;
-    if ((err = po_workspace(mode, prec, gsrc, gs, gtgt, gt, scalar ? dcur : nullptr, scalar ? dcur + gs : nullptr, ws))) return err;
+    if ((err = po_workspace(mode, prec, gs, gtgt, gt, ws))) return err;
     if (mode == PYPO_MODE_SCALAR) {
         err = launch_pack_scalar(prec, gsrc, gs, dcur, dcur + gs, sp.gmode, sp.n_cells[0],
-                                 sp.n_cells[1], packed, st);
+                                 sp.n_cells[1], packed, st, ws.near_ptr());
     } else {
         Bundle12 b;
         for (int q = 0; q < 12; q++) b.p[q] = dcur + q * (size_t)gs;
         err = launch_pack_sources(prec, gsrc, gs, b, sp.gmode, sp.n_cells[0], sp.n_cells[1], packed,
-                                  st, ws.cheb_ptr());
+                                  st, ws.cheb_ptr(), ws.near_ptr());
     }
     if (err) return err;
 
@@ -917,16 +913,13 @@ int pypo_hip_propagate_dev(int mode, void *res, const reflcontainer *cs, const r
     if (err) return err;
     PoWs ws;
     GridPtrs gsrc = grid_ptrs(*cs);
-    const arrC1 *sf = mode == PYPO_MODE_SCALAR ? (const arrC1 *)currents : nullptr;
-    if ((err = po_workspace(mode, precision, gsrc, gs, grid_ptrs(*ct), gt, sf ? sf->x : nullptr, sf ? sf->y : nullptr,
-                            ws)))
-        return err;
+    if ((err = po_workspace(mode, precision, gs, grid_ptrs(*ct), gt, ws))) return err;
     if (mode == PYPO_MODE_SCALAR) {
         const arrC1 *f = (const arrC1 *)currents;
-        err = launch_pack_scalar(precision, gsrc, gs, f->x, f->y, gmode, ncx, ncy, packed, st);
+        err = launch_pack_scalar(precision, gsrc, gs, f->x, f->y, gmode, ncx, ncy, packed, st, ws.near_ptr());
     } else {
         err = launch_pack_sources(precision, gsrc, gs, bundle12(*(const c2Bundle *)currents), gmode,
-                                  ncx, ncy, packed, st, ws.cheb_ptr());
+                                  ncx, ncy, packed, st, ws.cheb_ptr(), ws.near_ptr());
     }
     if (err) return err;
     err = launch_po(ws.plan, mode, precision, packed, gs, grid_ptrs(*ct), gt, k, epsilon, t_direction, res,
@@ -1009,10 +1002,7 @@ int pypo_hip_propagate_noalloc(int mode, void *res, const reflcontainer *cs, con
     const SumPlan plan = plan_cap_splits(plan_sum(mode, precision, gs, gt), gs, (int)std::min(fit, 1LL << 30));
     double *partial = (double *)((char *)base + pk);
     PoWs ws;
-    const arrC1 *sf = mode == PYPO_MODE_SCALAR ? (const arrC1 *)currents : nullptr;
-    if (cheb)
-        po_extra((char *)partial + wsb, mode, grid_ptrs(*cs), gs, grid_ptrs(*ct), gt, sf ? sf->x : nullptr,
-                 sf ? sf->y : nullptr, ws);
+    if (cheb) po_extra((char *)partial + wsb, mode, gs, grid_ptrs(*ct), gt, ws);
     PYPO_REQUIRE(partial_bytes(mode, plan, gt) <= wsb, ERR_ARG, "internal: split plan exceeds the scratch");
     hipStream_t st = (hipStream_t)stream;   // NULL: the default stream
     if ((err = begin_call(st))) return err;
@@ -1023,10 +1013,10 @@ int pypo_hip_propagate_noalloc(int mode, void *res, const reflcontainer *cs, con
     GridPtrs gsrc = grid_ptrs(*cs);
     if (mode == PYPO_MODE_SCALAR) {
         const arrC1 *f = (const arrC1 *)currents;
-        err = launch_pack_scalar(precision, gsrc, gs, f->x, f->y, gmode, ncx, ncy, base, st);
+        err = launch_pack_scalar(precision, gsrc, gs, f->x, f->y, gmode, ncx, ncy, base, st, ws.near_ptr());
     } else {
         err = launch_pack_sources(precision, gsrc, gs, bundle12(*(const c2Bundle *)currents), gmode, ncx,
-                                  ncy, base, st, ws.cheb_ptr());
+                                  ncy, base, st, ws.cheb_ptr(), ws.near_ptr());
     }
     if (err) return err;
     err = launch_po(plan, mode, precision, base, gs, grid_ptrs(*ct), gt, k, epsilon, t_direction, res, partial, wsb,

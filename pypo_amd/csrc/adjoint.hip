@@ -928,7 +928,7 @@ int launch_ff_power_grad(int precision, const GridPtrs &dish, int n_dish, int gm
     if (p.far_bytes) far = adj_far_carve(extra, precision, n_dish, ff, n_tgt);
     NearWs near;
     if (p.near_bytes)
-        near = near_cheb_carve(extra + p.far_bytes, PYPO_MODE_JM, feed, n_feed, dish, n_dish, nullptr, nullptr);
+        near = near_cheb_carve(extra + p.far_bytes, PYPO_MODE_JM, n_feed, dish, n_dish);
     int err;
     if (far.w.plan &&
         (err = launch_adj_far(precision, far, dish, n_dish, E, g, rev_scale, pc.prefactor, tg, st)))
@@ -940,7 +940,9 @@ int launch_ff_power_grad(int precision, const GridPtrs &dish, int n_dish, int gm
         hipLaunchKernelGGL(k_adj_targets<TgtRec32>, dim3(tb), dim3(256), 0, st, ff.x, ff.y, E, g, n_tgt,
                            rev_scale, pc.prefactor, (TgtRec32 *)tg, far.w.plan);
     PYPO_CHECK_LAUNCH();
-    if ((err = launch_pack_sources(precision, feed, n_feed, feed_cur, fgmode, fncx, fncy, fpk, st))) return err;
+    if ((err = launch_pack_sources(precision, feed, n_feed, feed_cur, fgmode, fncx, fncy, fpk, st, nullptr,
+                                   near.plan ? &near : nullptr)))
+        return err;
     void *feed64 = extra + p.far_bytes + p.near_bytes;
     if (near.plan && fp64) feed64 = fpk;
     if (near.plan && !fp64 && (err = launch_pack_sources(PYPO_PREC_FP64, feed, n_feed, feed_cur, fgmode, fncx, fncy, feed64, st)))

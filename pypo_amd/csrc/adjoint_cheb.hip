@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void k_adj_dish_meta(GridPtrs dish, int n, Til
         m.ax = c.ax; m.ay = c.ay; m.az = c.az; m.cos_half = c.cos_half;
         meta[blockIdx.x] = m;
     }
-    position_box(w, blockIdx.x, p, valid, scratch);
+    position_box(w.src_box, blockIdx.x, p, valid, scratch);
 }
 
 // Per target: arccos of its place along both axes, and A_t exp(-j t k c.r_t) (3

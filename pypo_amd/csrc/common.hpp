@@ -214,12 +214,15 @@ hipStream_t lib_stream(int *err);
 int launch_generate_grid(const reflparams &r, const GridPtrs &g, int n, const double *d_errs,
                          bool transform, bool spheric, hipStream_t st);
 
-// cheb: nullptr, or the workspace of a Chebyshev grid, whose boxes are filled.
+// cheb, near: nullptr, or the workspace of a Chebyshev grid, whose boxes are filled.
 struct ChebWs;
+struct NearWs;
 int launch_pack_sources(int precision, const GridPtrs &cs, int n_src, const Bundle12 &cur,
-                        int gmode, int ncx, int ncy, void *packed, hipStream_t st, const ChebWs *cheb = nullptr);
+                        int gmode, int ncx, int ncy, void *packed, hipStream_t st, const ChebWs *cheb = nullptr,
+                        const NearWs *near = nullptr);
 int launch_pack_scalar(int precision, const GridPtrs &cs, int n_src, const double *ur,
-                       const double *ui, int gmode, int ncx, int ncy, void *packed, hipStream_t st);
+                       const double *ui, int gmode, int ncx, int ncy, void *packed, hipStream_t st,
+                       const NearWs *near = nullptr);
 // Packed records plus (for the vector modes) one TileMeta per 256 sources.
 size_t packed_bytes(int mode, int precision, int n_src);
 
@@ -251,10 +254,9 @@ int tail_splits(long long blocks, long long tiles, int lo, int hi, long long slo
 // plan (plan_sum's, or one derived from it).  `res` points to a device-side
 // bundle struct of the mode's result type (c2Bundle / c4Bundle / c2rBundle /
 // arrC1) whose arrays are device memory.  cheb, near: workspace of the
-// Chebyshev grid of a far field (po_cheb.hpp; its boxes were filled by
-// launch_pack_sources) or of a near field (po_near_cheb.hpp), nullptr where it
-// is not tried.
-struct NearWs;
+// Chebyshev grid of a far field (po_cheb.hpp) or of a near field
+// (po_near_cheb.hpp), whose boxes the pack pass filled, nullptr where it is not
+// tried.
 int launch_po(const SumPlan &p, int mode, int precision, const void *packed, int n_src, const GridPtrs &ct,
               int n_tgt, double k, double epsilon, double t_dir, void *res, double *partial_ws, size_t ws_bytes,
               const ChebWs *cheb, const NearWs *near, hipStream_t st, bool time_it);

@@ -42,9 +42,8 @@ __device__ __forceinline__ void target_box(const ChebWs &w, int block, float *sc
     }
 }
 
-// Box of a tile's positions (this lane's: p), for the plan.
-__device__ __forceinline__ void position_box(const ChebWs &w, int tile, const double (&p)[3], bool valid,
-                                             float *scratch) {
+// Box [min x, y, z, max x, y, z] of a tile's positions (this lane's: p), for the plan.
+__device__ __forceinline__ void position_box(float *box, int tile, const double (&p)[3], bool valid, float *scratch) {
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const float x = (float)p[q];
@@ -53,8 +52,8 @@ __device__ __forceinline__ void position_box(const ChebWs &w, int tile, const do
         const float lo = block_min(valid ? (nan ? -INFINITY : x) : INFINITY, scratch);
         const float hi = -block_min(valid ? (nan ? -INFINITY : -x) : INFINITY, scratch);
         if (threadIdx.x == 0) {
-            w.src_box[6 * tile + q] = lo;
-            w.src_box[6 * tile + 3 + q] = hi;
+            box[6 * tile + q] = lo;
+            box[6 * tile + 3 + q] = hi;
         }
     }
 }

@@ -10,37 +10,20 @@
 namespace pypo {
 namespace {
 
-// Boxes of kNearBox sources (first) or targets per workgroup, in FP32.
-__global__ __launch_bounds__(256) void k_near_boxes(NearWs w) {
-    __shared__ float scratch[4];
-    const bool tgt = (int)blockIdx.x >= w.src_blocks();
-    const int base = (blockIdx.x - (tgt ? w.src_blocks() : 0)) * kNearBox, n = tgt ? w.n_tgt : w.n_src;
-    const double *p[3] = {tgt ? w.tx : w.sx, tgt ? w.ty : w.sy, tgt ? w.tz : w.sz};
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {INFINITY, INFINITY, INFINITY}, bad = 0.f;
+constexpr float kNearCompact = 1.f / 3.f;   // largest rho / R of a plan that is on
+constexpr float kNearWide = 1.5f;           // largest |a|, |b|
+
+// Wave-wide minima of N values, step by step so that the exchanges of one step
+// are in flight together.
+template <int N>
+__device__ __forceinline__ void wave_minima(float (&v)[N]) {
 #pragma unroll
-    for (int j = 0; j < kNearBox / 256; j++) {
-        const int i = base + j * 256 + threadIdx.x;
-        if (i >= n) break;
+    for (int o = 32; o >= 1; o >>= 1) {
+        float x[N];
 #pragma unroll
-        for (int q = 0; q < 3; q++) {
-            const float x = (float)p[q][i];
-            lo[q] = fminf(lo[q], x);
-            hi[q] = fminf(hi[q], -x);
-            if (!(fabsf(x) < 1e30f)) bad = 1.f;
-        }
-        // a scalar field's infinities keep the sums' own infinities and NaN
-        if (!tgt && w.u && !(fabs(w.u[i]) < 1e300 && fabs(w.v[i]) < 1e300)) bad = 1.f;
-    }
-    bad = -block_min(-bad, scratch);
+        for (int q = 0; q < N; q++) x[q] = __shfl_xor(v[q], o, 64);
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-        lo[q] = block_min(lo[q], scratch);
-        hi[q] = -block_min(hi[q], scratch);
-    }
-    if (threadIdx.x == 0) {
-        float *o = w.box + 6 * blockIdx.x;
-        for (int q = 0; q < 3; q++) { o[q] = lo[q]; o[3 + q] = hi[q]; }
-        if (bad > 0.f) o[0] = __builtin_nanf("");
+        for (int q = 0; q < N; q++) v[q] = fminf(v[q], x[q]);
     }
 }
 
@@ -59,8 +42,7 @@ __device__ void near_extent(const float *box, int b0, int b1, float (*red)[9], d
             if (!(fabsf(x) < 1e30f)) v[2 * N] = -1.f;
             v[q] = fminf(v[q], x);
         }
-#pragma unroll
-    for (int q = 0; q <= 2 * N; q++) v[q] = wave_min(v[q]);
+    wave_minima(v);
     __syncthreads();
     if (lane == 0)
 #pragma unroll
@@ -97,121 +79,31 @@ __device__ void near_frame(const double (&c)[3], const double (&tc)[3], double (
     e[1][2] = d[0] * e[0][1] - d[1] * e[0][0];
 }
 
-// One workgroup: the frame, and the quadratic surface through 256 of the
-// targets (scattered over their order by the golden ratio).  Any coefficients
-// are right, good ones make s small: a singular fit drops terms.
-__global__ __launch_bounds__(256) void k_near_frame(NearWs w) {
-    __shared__ float red[4][9];
-    __shared__ double sum[4][32];
-    __shared__ float scratch[4];
-    double c[3], half[3], tc[3], th[3], e[3][3];
-    bool bad_s, bad_t;
-    near_extent<3>(w.box, 0, w.src_blocks(), red, c, half, bad_s);
-    near_extent<3>(w.box, w.src_blocks(), w.src_blocks() + w.tgt_blocks(), red, tc, th, bad_t);
-    near_frame(c, tc, e);
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const double g = tid * 0.6180339887498949;
-    const int t = min(w.n_tgt - 1, (int)((g - floor(g)) * w.n_tgt));
-    const double u[3] = {w.tx[t] - c[0], w.ty[t] - c[1], w.tz[t] - c[2]};
-    const double s = 1.0 / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-    double a, b, theta;
-    near_coords(e, u, a, b, theta);
-    const float la = block_min((float)a, scratch), ha = -block_min(-(float)a, scratch);
-    const float lb = block_min((float)b, scratch), hb = -block_min(-(float)b, scratch);
-    const double fa = 0.5 * ((double)la + ha), fb = 0.5 * ((double)lb + hb);
-    const double ga = 2.0 / fmax((double)ha - la, 1e-9), gb = 2.0 / fmax((double)hb - lb, 1e-9);
-    const double x = (a - fa) * ga, y = (b - fb) * gb;
-    const double f[7] = {1.0, x, y, x * x, x * y, y * y, s};
-    // normal equations: the 27 products, summed over the workgroup
-    int k = 0;
-#pragma unroll
-    for (int i = 0; i < 6; i++)
-#pragma unroll
-        for (int j = i; j < 7; j++, k++) {
-            double p = f[i] * f[j];
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) p += __shfl_xor(p, o, 64);
-            if (lane == 0) sum[wv][k] = p;
-        }
+// Block-wide minima of N values; red: [4][N].
+template <int N>
+__device__ __forceinline__ void block_minima(float (&v)[N], float (*red)[9]) {
+    static_assert(N <= 9, "rows of red");
+    wave_minima(v);
     __syncthreads();
-    if (tid) return;
-    double m[6][7];
-    k = 0;
+    if ((threadIdx.x & 63) == 0)
 #pragma unroll
-    for (int i = 0; i < 6; i++)
+        for (int q = 0; q < N; q++) red[threadIdx.x >> 6][q] = v[q];
+    __syncthreads();
 #pragma unroll
-        for (int j = i; j < 7; j++, k++) {
-            m[i][j] = sum[0][k] + sum[1][k] + sum[2][k] + sum[3][k];
-            if (j < 6) m[j][i] = m[i][j];
-        }
-    // Gauss-Jordan with the diagonal as pivot (symmetric positive semi-definite)
-    bool used[6];
-#pragma unroll
-    for (int p = 0; p < 6; p++) {
-        used[p] = m[p][p] > 1e-9 * 256.0;
-        if (!used[p]) continue;
-        const double inv = 1.0 / m[p][p];
-#pragma unroll
-        for (int j = 0; j < 7; j++) m[p][j] *= inv;
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            if (i == p) continue;
-            const double q = m[i][p];
-#pragma unroll
-            for (int j = 0; j < 7; j++) m[i][j] -= q * m[p][j];
-        }
-    }
-    NearPlan &pl = *w.plan;
-    pl.on = !bad_s && !bad_t;
-    for (int q = 0; q < 3; q++) {
-        pl.c[q] = c[q];
-        for (int r = 0; r < 3; r++) pl.e[q][r] = e[q][r];
-        pl.ext[q] = fabs(e[q][0]) * half[0] + fabs(e[q][1]) * half[1] + fabs(e[q][2]) * half[2];
-    }
-    pl.ext[3] = sqrt(half[0] * half[0] + half[1] * half[1] + half[2] * half[2]);
-#pragma unroll
-    for (int q = 0; q < 6; q++) pl.fit[q] = used[q] ? m[q][6] : 0.0;
-    pl.fa = fa; pl.fb = fb; pl.ga = ga; pl.gb = gb;
+    for (int q = 0; q < N; q++) v[q] = fminf(fminf(red[0][q], red[1][q]), fminf(red[2][q], red[3][q]));
 }
 
-// Box of kNearBox targets per workgroup in (a, b, 1/R, s), their largest
-// theta, and how far a wave's 64 consecutive targets spread.
-__global__ __launch_bounds__(256) void k_near_cones(NearWs w) {
-    __shared__ float scratch[4];
-    const NearPlan &pl = *w.plan;
-    float v[9], ea = 0.f, eb = 0.f, waves = 0.f;
-#pragma unroll
-    for (int q = 0; q < 9; q++) v[q] = INFINITY;
-#pragma unroll 1
-    for (int j = 0; j < kNearBox / 256; j++) {
-        const int t = blockIdx.x * kNearBox + j * 256 + threadIdx.x;
-        if (__ballot(t < w.n_tgt) == 0ull) break;
-        const int i = min(t, w.n_tgt - 1);
-        const double u[3] = {w.tx[i] - pl.c[0], w.ty[i] - pl.c[1], w.tz[i] - pl.c[2]};
-        const double r = 1.0 / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-        double a, b, theta;
-        near_coords(pl.e, u, a, b, theta);
-        const float fa = (float)a, fb = (float)b, fr = (float)r, fs = (float)(r - pl.surface(a, b));
-        v[0] = fminf(v[0], fa); v[4] = fminf(v[4], -fa);
-        v[1] = fminf(v[1], fb); v[5] = fminf(v[5], -fb);
-        v[2] = fminf(v[2], fr); v[6] = fminf(v[6], -fr);
-        v[3] = fminf(v[3], fs); v[7] = fminf(v[7], -fs);
-        v[8] = fminf(v[8], -(float)theta);
-        ea -= wave_min(fa) + wave_min(-fa);
-        eb -= wave_min(fb) + wave_min(-fb);
-        waves += 1.f;
-    }
-#pragma unroll
-    for (int q = 0; q < 9; q++) v[q] = block_min(v[q], scratch);
-    const bool first = (threadIdx.x & 63) == 0;
-    ea = block_sum(first ? ea : 0.f, scratch);
-    eb = block_sum(first ? eb : 0.f, scratch);
-    waves = block_sum(first ? waves : 0.f, scratch);
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < 8; q++) w.cone[8 * blockIdx.x + q] = q < 4 ? v[q] : -v[q];
-        float *o = w.theta + 4 * blockIdx.x;
-        o[0] = -v[8]; o[1] = ea; o[2] = eb; o[3] = waves;
-    }
+// A tile of sources that may not light all of the cone, or carries infinite currents.
+__device__ __forceinline__ bool near_tile_off(const TileMeta &t, const Cone &cone) {
+    return !(t.cmax < INFINITY) || cones_may_shadow(t.ax, t.ay, t.az, t.cos_half, cone);
+}
+
+__device__ __forceinline__ Cone near_cone(const double (&axis)[3], float theta, float near) {
+    Cone cone;
+    cone.ax = (float)axis[0]; cone.ay = (float)axis[1]; cone.az = (float)axis[2];
+    const float ang = theta + asinf(near);   // widened by the sources' parallax
+    cone.cos_half = ang < 1.57f ? cosf(ang) : -1.f;
+    return cone;
 }
 
 constexpr int kNearSmall = 24;
@@ -263,7 +155,173 @@ __device__ float near_axis(const NearIn &in, float h, float x, float y, float z,
     return n;
 }
 
-// One workgroup: decide, choose the patches, write the plan.
+// Rates and radial nodes of a box: half widths and largest |a|, |b|, the
+// sources' half extents along the frame and rho, the largest 1 / R, the half
+// width in s and the surface's slope.
+struct NearGeo {
+    float ha, hb, la, lb, ex, ey, ez, grow, tilt, cap;
+    int nr;
+};
+__device__ __forceinline__ NearGeo near_geo(const NearIn &in, float ha, float hb, float la, float lb,
+                                            const float (&ext)[4], float r1, float hs, float slope) {
+    NearGeo g{ha, hb, la, lb, ext[0], ext[1], ext[2]};
+    const float rho = ext[3], near = rho * r1;
+    g.grow = 1.f / (1.f - fminf(near, 0.5f));
+    // radial phase and amplitude rates per unit of s: those that vanish with the
+    // sources' extent, and with the dyadic's own
+    const float smooth = 1.1f * g.grow * g.grow * in.kabs * 0.5f * rho * rho + 2.f * rho * g.grow;
+    const float radial = smooth + in.dyadic;
+    g.tilt = radial * slope;
+    g.cap = fminf(1.5f, 0.8f * acoshf(1.f / near));
+    // no further than four fifths of the way to the singularity at s = 1 / rho
+    const float far = 1.f + fmaxf(0.f, (0.8f / rho - r1) / hs);
+    const float least = ceilf(in.log_eps / __logf(far + sqrtf(far * far - 1.f)));
+    // the dyadic is a polynomial of degree two in s: two more nodes always do
+    g.nr = (int)fminf(fmaxf(near_count(smooth * hs, in), least) + 2.f, fmaxf(near_count(radial * hs, in), least));
+    return g;
+}
+
+// The nodes of choice `at` of the patches (16 x 16), and the issue cycles of 64
+// lanes of their sums and of the series at the targets (7 cycles an FMA with its
+// scalar loads, measured) where a wave meets one patch; false: too many nodes.
+__device__ __forceinline__ bool near_cost(const NearIn &in, const NearGeo &g, int at, float &na, float &nb, float &nodes,
+                                          float &one) {
+    const int pa = at / kNearMaxPatches + 1, pb = at % kNearMaxPatches + 1;
+    na = near_axis(in, g.ha / pa, g.ex, g.ey, g.ez, g.tilt, g.la, g.lb, g.grow, g.cap);
+    nb = near_axis(in, g.hb / pb, g.ey, g.ex, g.ez, g.tilt, g.lb, g.la, g.grow, g.cap);
+    const float each = na * nb * g.nr, all = each * pa * pb;
+    nodes = ceilf(all * (1.f / 256.f)) * 4.f * in.n_src * in.pair_cycles;
+    one = in.n_tgt * (1.f / 64.f) * each * (in.rows + 1) * in.series_cycles;
+    return na <= kNearMaxAxis && nb <= kNearMaxAxis && g.nr <= kNearMaxRadial && all <= kNearMaxNodes && all <= in.n_tgt;
+}
+
+// Whether that pays against the sums at the targets.
+__device__ __forceinline__ bool near_pays(const NearIn &in, float cost) {
+    return cost + in.fixed_cycles < 0.7f * (in.n_tgt * (1.f / 64.f) * (float)in.n_src * in.direct_cycles);
+}
+
+// One workgroup: the frame, and the quadratic surface through 256 of the
+// targets (scattered over their order by the golden ratio).  Any coefficients
+// are right, good ones make s small: a singular fit drops terms.  Where those
+// targets alone already turn the plan off (too near, too wide, in shadow, too
+// many nodes for their box), so would all of them: the kernels behind see that and return.
+static_assert(kNearMaxPatches * kNearMaxPatches == 256, "one choice a lane");
+__global__ __launch_bounds__(256) void k_near_frame(NearIn in, NearWs w) {
+    __shared__ float red[4][9];
+    __shared__ double sum[4][32], surface[6];
+    double c[3], half[3], tc[3], th[3], e[3][3];
+    bool bad, bad_t;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    if (tid == 0) w.plan->on = 0;
+    const double g = tid * 0.6180339887498949;
+    const int t = min(w.n_tgt - 1, (int)((g - floor(g)) * w.n_tgt));
+    const double p[3] = {w.tx[t], w.ty[t], w.tz[t]};
+    near_extent<3>(w.box, 0, w.src_tiles(), red, c, half, bad);
+    near_extent<3>(w.box, w.src_tiles(), w.src_tiles() + w.tgt_blocks(), red, tc, th, bad_t);
+    if (bad || bad_t) return;
+    near_frame(c, tc, e);
+    const double u[3] = {p[0] - c[0], p[1] - c[1], p[2] - c[2]};
+    const double s = 1.0 / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+    const double rho = sqrt(half[0] * half[0] + half[1] * half[1] + half[2] * half[2]);
+    double a, b, theta;
+    near_coords(e, u, a, b, theta);
+    float v[6] = {(float)a, (float)b, -(float)a, -(float)b, -(float)theta, -(float)s};
+    block_minima(v, red);
+    const float la = v[0], lb = v[1], ha = -v[2], hb = -v[3], near = (float)rho * -v[5];
+    bool off = !(near <= kNearCompact && fmaxf(fmaxf(-la, ha), fmaxf(-lb, hb)) <= kNearWide);
+    if (in.meta && !off) {
+        const Cone cone = near_cone(e[2], -v[4], near);
+        for (int i = tid; i < in.n_tiles; i += 256) off |= near_tile_off(in.meta[i], cone);
+    }
+    if (__syncthreads_or(off)) return;
+    const double fa = 0.5 * ((double)la + ha), fb = 0.5 * ((double)lb + hb);
+    const double ga = 2.0 / fmax((double)ha - la, 1e-9), gb = 2.0 / fmax((double)hb - lb, 1e-9);
+    const double x = (a - fa) * ga, y = (b - fb) * gb;
+    const double f[7] = {1.0, x, y, x * x, x * y, y * y, s};
+    // normal equations: the 27 products, summed over the workgroup
+    double prod[27];
+    int k = 0;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+#pragma unroll
+        for (int j = i; j < 7; j++, k++) prod[k] = f[i] * f[j];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        double x[27];
+#pragma unroll
+        for (int q = 0; q < 27; q++) x[q] = __shfl_xor(prod[q], o, 64);
+#pragma unroll
+        for (int q = 0; q < 27; q++) prod[q] += x[q];
+    }
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < 27; q++) sum[wv][q] = prod[q];
+    __syncthreads();
+    if (tid == 0) {
+        double m[6][7];
+        k = 0;
+#pragma unroll
+        for (int i = 0; i < 6; i++)
+#pragma unroll
+            for (int j = i; j < 7; j++, k++) {
+                m[i][j] = sum[0][k] + sum[1][k] + sum[2][k] + sum[3][k];
+                if (j < 6) m[j][i] = m[i][j];
+            }
+        // Gauss-Jordan with the diagonal as pivot (symmetric positive semi-definite)
+        bool used[6];
+#pragma unroll
+        for (int p = 0; p < 6; p++) {
+            used[p] = m[p][p] > 1e-9 * 256.0;
+            if (!used[p]) continue;
+            const double inv = 1.0 / m[p][p];
+#pragma unroll
+            for (int j = 0; j < 7; j++) m[p][j] *= inv;
+#pragma unroll
+            for (int i = 0; i < 6; i++) {
+                if (i == p) continue;
+                const double q = m[i][p];
+#pragma unroll
+                for (int j = 0; j < 7; j++) m[i][j] -= q * m[p][j];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 6; q++) surface[q] = used[q] ? m[q][6] : 0.0;
+    }
+    __syncthreads();
+    double ext[4];
+    for (int q = 0; q < 3; q++)
+        ext[q] = fabs(e[q][0]) * half[0] + fabs(e[q][1]) * half[1] + fabs(e[q][2]) * half[2];
+    ext[3] = rho;
+    {
+        // the plan's cost for these targets alone, no slope, patches met one by one
+        double res = s;
+#pragma unroll
+        for (int q = 0; q < 6; q++) res -= surface[q] * f[q];
+        float r[4] = {(float)res, -(float)res, (float)s, -(float)s};
+        block_minima(r, red);
+        const float hs = fmaxf(fminf(-r[1] - r[0], -r[3] - r[2]) * 0.5f, -1e-7f * r[3]);
+        const float ex[4] = {(float)ext[0], (float)ext[1], (float)ext[2], (float)ext[3]};
+        const NearGeo geo = near_geo(in, fmaxf(0.5f * (ha - la), 1e-6f), fmaxf(0.5f * (hb - lb), 1e-6f), fmaxf(-la, ha),
+                                     fmaxf(-lb, hb), ex, -r[3], hs, 0.f);
+        float na, nb, nodes, one;
+        const bool ok = near_cost(in, geo, tid, na, nb, nodes, one);
+        if (!__syncthreads_or(ok && near_pays(in, nodes + one))) return;
+    }
+    if (tid) return;
+    NearPlan &pl = *w.plan;
+    pl.on = 1;
+    for (int q = 0; q < 3; q++) {
+        pl.c[q] = c[q];
+        for (int r = 0; r < 3; r++) pl.e[q][r] = e[q][r];
+    }
+    for (int q = 0; q < 4; q++) pl.ext[q] = ext[q];
+    for (int q = 0; q < 6; q++) pl.fit[q] = surface[q];
+    pl.fa = fa; pl.fb = fb; pl.ga = ga; pl.gb = gb;
+}
+
+// One workgroup: decide, choose the patches, write the plan.  A kernel of its
+// own: as the last workgroup of k_near_cones, behind a fence in each of them, it
+// saved a launch but took 20 us more at 1 002 001 targets.
 __global__ __launch_bounds__(1024) void k_near_plan(NearIn in, NearWs w) {
     __shared__ float red[16][9];
     __shared__ float spread[16][4];
@@ -274,6 +332,7 @@ __global__ __launch_bounds__(1024) void k_near_plan(NearIn in, NearWs w) {
     const int tid = threadIdx.x, lane = tid & 63;
     double mid[4], half[4];
     bool bad;
+    if (!w.plan->on) return;
     if (tid == 0) {
         pl = *w.plan;
         best = ~0ull;
@@ -323,59 +382,36 @@ __global__ __launch_bounds__(1024) void k_near_plan(NearIn in, NearWs w) {
         }
     }
     const float near = rho * r1;
-    bool on = pl.on && !bad && la <= 1.5f && lb <= 1.5f && r0 > 0.f && near <= 1.f / 3.f;
+    bool on = !bad && la <= kNearWide && lb <= kNearWide && r0 > 0.f && near <= kNearCompact;
     if (on && in.meta) {
-        // every source lights every target: cone of the targets from c, widened
-        // by the sources' parallax
-        Cone cone;
-        cone.ax = (float)pl.e[2][0]; cone.ay = (float)pl.e[2][1]; cone.az = (float)pl.e[2][2];
-        const float ang = theta + asinf(near);
-        cone.cos_half = ang < 1.57f ? cosf(ang) : -1.f;
-        for (int i = tid; i < in.n_tiles; i += 1024) {
-            const TileMeta t = in.meta[i];
-            if (!(t.cmax < INFINITY) || cones_may_shadow(t.ax, t.ay, t.az, t.cos_half, cone)) shadow = 1;
-        }
+        // every source lights every target
+        const Cone cone = near_cone(pl.e[2], theta, near);
+        for (int i = tid; i < in.n_tiles; i += 1024)
+            if (near_tile_off(in.meta[i], cone)) shadow = 1;
     }
     __syncthreads();
     on = on && !shadow;
     const float ha = fmaxf((float)half[0], 1e-6f), hb = fmaxf((float)half[1], 1e-6f);
     const float hs = fmaxf((float)half[fit ? 3 : 2], 1e-7f * r1);
-    const float grow = 1.f / (1.f - fminf(near, 0.5f));
-    // radial phase and amplitude rates per unit of s: those that vanish with the
-    // sources' extent, and with the dyadic's own
-    const float smooth = 1.1f * grow * grow * in.kabs * 0.5f * rho * rho + 2.f * rho * grow;
-    const float radial = smooth + in.dyadic, tilt = radial * slope;
-    const float cap = fminf(1.5f, 0.8f * acoshf(1.f / near));
     int nr = 0;
     if (on) {
-        // no further than four fifths of the way to the singularity at s = 1 / rho
-        const float far = 1.f + fmaxf(0.f, (0.8f / rho - r1) / hs);
-        const float least = ceilf(in.log_eps / __logf(far + sqrtf(far * far - 1.f)));
-        // the dyadic is a polynomial of degree two in s: two more nodes always do
-        nr = (int)fminf(fmaxf(near_count(smooth * hs, in), least) + 2.f, fmaxf(near_count(radial * hs, in), least));
+        const float ext[4] = {ex, ey, ez, rho};
+        const NearGeo geo = near_geo(in, ha, hb, la, lb, ext, r1, hs, slope);
+        nr = geo.nr;
         if (tid < kNearMaxPatches * kNearMaxPatches) {
-            const int pa = tid / kNearMaxPatches + 1, pb = tid % kNearMaxPatches + 1;
-            const float na = near_axis(in, ha / pa, ex, ey, ez, tilt, la, lb, grow, cap);
-            const float nb = near_axis(in, hb / pb, ey, ex, ez, tilt, lb, la, grow, cap);
-            const float each = na * nb * nr, all = each * pa * pb;
+            float na, nb, nodes, one;
+            const bool ok = near_cost(in, geo, tid, na, nb, nodes, one);
             nodes_a[tid] = (unsigned short)fminf(na, 1e4f);
             nodes_b[tid] = (unsigned short)fminf(nb, 1e4f);
-            if (na <= kNearMaxAxis && nb <= kNearMaxAxis && nr <= kNearMaxRadial && all <= kNearMaxNodes &&
-                all <= in.n_tgt) {
-                // issue cycles of 64 lanes: the node sums, and the series at the
-                // targets (7 cycles an FMA with its scalar loads, measured) for
-                // every patch a wave meets
-                const float nodes = ceilf(all * (1.f / 256.f)) * 4.f * in.n_src * in.pair_cycles;
-                const float one = in.n_tgt * (1.f / 64.f) * each * (in.rows + 1) * in.series_cycles;
-                const float met = (1.f + ea * pa / (2.f * ha)) * (1.f + eb * pb / (2.f * hb));
-                const float plain = one * (pa * pb > 1 ? met : 1.f);
-                const float sorted = in.sort_cycles > 0.f ? one * 1.1f + in.sort_cycles : INFINITY;
-                const float direct = in.n_tgt * (1.f / 64.f) * (float)in.n_src * in.direct_cycles;
-                const float cost = nodes + fminf(plain, sorted);
-                if (cost + in.fixed_cycles < 0.7f * direct)
-                    atomicMin(&best, (unsigned long long)__float_as_uint(cost) << 32 | (sorted < plain ? 1u << 31 : 0u) |
-                                         (unsigned)tid);
-            }
+            const int pa = tid / kNearMaxPatches + 1, pb = tid % kNearMaxPatches + 1;
+            // a wave's targets meet several patches in grid order
+            const float met = (1.f + ea * pa / (2.f * ha)) * (1.f + eb * pb / (2.f * hb));
+            const float plain = one * (pa * pb > 1 ? met : 1.f);
+            const float sorted = in.sort_cycles > 0.f ? one * 1.1f + in.sort_cycles : INFINITY;
+            const float cost = nodes + fminf(plain, sorted);
+            if (ok && near_pays(in, cost))
+                atomicMin(&best, (unsigned long long)__float_as_uint(cost) << 32 | (sorted < plain ? 1u << 31 : 0u) |
+                                     (unsigned)tid);
         }
     }
     __syncthreads();
@@ -423,6 +459,47 @@ __global__ __launch_bounds__(1024) void k_near_plan(NearIn in, NearWs w) {
         pl.chunk = ct * TILE;
         pl.splits = (in.n_tiles + ct - 1) / ct;
         *w.plan = pl;
+    }
+}
+
+// Box of kNearBox targets per workgroup in (a, b, 1/R, s), their largest
+// theta, and how far a wave's 64 consecutive targets spread.
+__global__ __launch_bounds__(256) void k_near_cones(NearWs w) {
+    __shared__ float scratch[4];
+    __shared__ float red[4][9];
+    const NearPlan &pl = *w.plan;
+    if (!pl.on) return;
+    float v[9], ea = 0.f, eb = 0.f, waves = 0.f;
+#pragma unroll
+    for (int q = 0; q < 9; q++) v[q] = INFINITY;
+#pragma unroll 1
+    for (int j = 0; j < kNearBox / 256; j++) {
+        const int t = blockIdx.x * kNearBox + j * 256 + threadIdx.x;
+        if (__ballot(t < w.n_tgt) == 0ull) break;
+        const int i = min(t, w.n_tgt - 1);
+        const double u[3] = {w.tx[i] - pl.c[0], w.ty[i] - pl.c[1], w.tz[i] - pl.c[2]};
+        const double r = 1.0 / sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        double a, b, theta;
+        near_coords(pl.e, u, a, b, theta);
+        const float fa = (float)a, fb = (float)b, fr = (float)r, fs = (float)(r - pl.surface(a, b));
+        v[0] = fminf(v[0], fa); v[4] = fminf(v[4], -fa);
+        v[1] = fminf(v[1], fb); v[5] = fminf(v[5], -fb);
+        v[2] = fminf(v[2], fr); v[6] = fminf(v[6], -fr);
+        v[3] = fminf(v[3], fs); v[7] = fminf(v[7], -fs);
+        v[8] = fminf(v[8], -(float)theta);
+        ea -= wave_min(fa) + wave_min(-fa);
+        eb -= wave_min(fb) + wave_min(-fb);
+        waves += 1.f;
+    }
+    block_minima(v, red);
+    const bool first = (threadIdx.x & 63) == 0;
+    ea = block_sum(first ? ea : 0.f, scratch);
+    eb = block_sum(first ? eb : 0.f, scratch);
+    waves = block_sum(first ? waves : 0.f, scratch);
+    if (threadIdx.x == 0) {
+        for (int q = 0; q < 8; q++) w.cone[8 * blockIdx.x + q] = q < 4 ? v[q] : -v[q];
+        float *o = w.theta + 4 * blockIdx.x;
+        o[0] = -v[8]; o[1] = ea; o[2] = eb; o[3] = waves;
     }
 }
 
@@ -618,14 +695,14 @@ constexpr int kNearSortTargets = 200000;
 }  // namespace
 
 // Tried where the sums at the targets take 300 us or more, 500 us with E: the
-// passes around them are some 60 us, 50 us where the plan stays off (with E it
-// stayed off for four of seven drawn calls of 300 to 500 us, 388 -> 437 us,
-// and took 548 to 232 and 601 to 311 us).  From 1 ms only in FP64 (its node
-// counts seldom pay below: 961 sources -> 90 300 targets stayed off, 0.62 ->
-// 0.67 ms), and for fewer sources than five times a patch's series costs at a
+// passes around them are some 60 us where the plan is on.  Off, they are 5 to 15
+// us where 256 targets show that (too near, too wide, in shadow: JM 745 -> 748 us,
+// EH 1046 -> 1053, scalar 366 -> 381) and 22 where their box asks for too many
+// nodes (JM 549 -> 571, scalar 352 -> 376; 45 without the early word).  From 1 ms only in
+// FP64 (its node counts seldom pay below: 961 sources -> 90 300 targets stayed
+// off), and for fewer sources than five times a patch's series costs at a
 // target at the node counts that a wavelength across a patch takes, 13^2 x 2
-// in three patches a wave (529 sources -> 344 874 targets with E: off, 661 ->
-// 720 us).
+// in three patches a wave.
 bool near_cheb_try(int mode, int precision, int n_src, int n_tgt) {
     const double cycles = pair_cycles(mode, precision);
     const double us = (double)n_src * n_tgt / 64 * cycles / kSimdHz * 1e6;
@@ -636,8 +713,8 @@ bool near_cheb_try(int mode, int precision, int n_src, int n_tgt) {
 
 size_t near_cheb_bytes(int mode, int n_src, int n_tgt) {
     const size_t cap = std::min(kNearMaxNodes, n_tgt);
-    const size_t sb = (n_src + kNearBox - 1) / kNearBox, tb = (n_tgt + kNearBox - 1) / kNearBox;
-    size_t b = 1024 + up256((sb + tb) * 6 * sizeof(float)) + up256(tb * 12 * sizeof(float)) +
+    const size_t tb = (n_tgt + kNearBox - 1) / kNearBox;
+    size_t b = 1024 + up256((n_tiles(n_src) + tb) * 6 * sizeof(float)) + up256(tb * 12 * sizeof(float)) +
                up256((3 + 2 * (size_t)near_rows(mode)) * cap * sizeof(double));
     if (n_tgt >= kNearSortTargets)
         b += up256((size_t)n_tgt * 8) +
@@ -645,20 +722,18 @@ size_t near_cheb_bytes(int mode, int n_src, int n_tgt) {
     return b;
 }
 
-NearWs near_cheb_carve(void *base, int mode, const GridPtrs &cs, int n_src, const GridPtrs &ct, int n_tgt,
-                       const double *u, const double *v) {
+NearWs near_cheb_carve(void *base, int mode, int n_src, const GridPtrs &ct, int n_tgt) {
     static_assert(sizeof(NearPlan) <= 1024, "room of the plan");
     const size_t cap = std::min(kNearMaxNodes, n_tgt);
     char *b = (char *)base;
     NearWs w;
-    w.sx = cs.x; w.sy = cs.y; w.sz = cs.z; w.u = u; w.v = v;
     w.tx = ct.x; w.ty = ct.y; w.tz = ct.z;
     w.n_src = n_src; w.n_tgt = n_tgt;
     const size_t tb = w.tgt_blocks();
     w.plan = (NearPlan *)b;
     b += 1024;
     w.box = (float *)b;
-    b += up256((w.src_blocks() + tb) * 6 * sizeof(float));
+    b += up256((w.src_tiles() + tb) * 6 * sizeof(float));
     w.cone = (float *)b;
     w.theta = w.cone + 8 * tb;
     b += up256(tb * 12 * sizeof(float));
@@ -680,12 +755,6 @@ NearWs near_cheb_carve(void *base, int mode, const GridPtrs &cs, int n_src, cons
 int launch_near_cheb_plan(int mode, int precision, int sums, const SumPlan &p, const TileMeta *meta, int n_src,
                           double kabs, size_t partial_bytes, double direct_cycles, const NearWs &w, hipStream_t st) {
     const bool f64 = precision == PYPO_PREC_FP64;
-    hipLaunchKernelGGL(k_near_boxes, dim3(w.src_blocks() + w.tgt_blocks()), dim3(256), 0, st, w);
-    PYPO_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_near_frame, dim3(1), dim3(256), 0, st, w);
-    PYPO_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_near_cones, dim3(w.tgt_blocks()), dim3(256), 0, st, w);
-    PYPO_CHECK_LAUNCH();
     NearIn in;
     in.meta = mode == PYPO_MODE_SCALAR ? nullptr : meta;
     in.n_tiles = n_tiles(n_src);
@@ -711,6 +780,10 @@ int launch_near_cheb_plan(int mode, int precision, int sums, const SumPlan &p, c
     in.series_cycles = (w.nodes_only ? 18.f : 7.f) * std::max(1.f, 2048.f * 64 / w.n_tgt);
     in.fixed_cycles = (float)((w.nodes_only ? 90e-6 : 40e-6) * kSimdHz);
     in.sort_cycles = w.slot ? (float)((15e-6 + 25e-12 * w.n_tgt) * kSimdHz) : 0.f;
+    hipLaunchKernelGGL(k_near_frame, dim3(1), dim3(256), 0, st, in, w);
+    PYPO_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_near_cones, dim3(w.tgt_blocks()), dim3(256), 0, st, w);
+    PYPO_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_near_plan, dim3(1), dim3(1024), 0, st, in, w);
     PYPO_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_near_nodes, dim3(64), dim3(256), 0, st, w);

@@ -55,7 +55,7 @@ constexpr int kNearMaxNodes = 65536;   // all patches together
 constexpr int kNearMaxAxis = 96;       // na, nb
 constexpr int kNearMaxRadial = 24;     // nr
 constexpr int kNearMaxPatches = 16;    // per axis
-constexpr int kNearBox = 1024;         // points per workgroup of the box passes
+constexpr int kNearBox = 1024;         // targets per workgroup of the box pass
 constexpr int kNearBin = 4096;         // targets per workgroup that counts them by patch
 
 struct NearPlan {
@@ -77,7 +77,7 @@ struct NearPlan {
 // Workspace of one propagation, behind the split partials, and its grids.
 struct NearWs {
     NearPlan *plan = nullptr;          // nullptr: not tried
-    float *box = nullptr;              // [source blocks, target blocks][6]: min x, y, z, max x, y, z (NaN: not finite)
+    float *box = nullptr;              // [source tile, then target block][6]: min x, y, z, max x, y, z (not finite: off)
     float *cone = nullptr;             // [target block][8]: min a, b, 1/R, s, max a, b, 1/R, s
     float *theta = nullptr;            // [target block][4]: largest theta, summed extents a, b of waves, waves
     double *x = nullptr, *y = nullptr, *z = nullptr;   // nodes
@@ -86,19 +86,16 @@ struct NearWs {
     unsigned *slot = nullptr;          // [target]: patch << 16 | rank in its bin; nullptr: no sorting
     int *count = nullptr;              // [patch][bin]: counts, then first positions
     int *perm = nullptr;               // [n_tgt] targets patch by patch
-    const double *sx = nullptr, *sy = nullptr, *sz = nullptr, *u = nullptr, *v = nullptr;   // sources; scalar field
-    const double *tx = nullptr, *ty = nullptr, *tz = nullptr;                               // targets
+    const double *tx = nullptr, *ty = nullptr, *tz = nullptr;   // targets
     int n_src = 0, n_tgt = 0;
     bool nodes_only = false;           // the sum kernel works on nodes or not at all
-    __host__ __device__ int src_blocks() const { return (n_src + kNearBox - 1) / kNearBox; }
+    __host__ __device__ int src_tiles() const { return (n_src + 255) / 256; }
     __host__ __device__ int tgt_blocks() const { return (n_tgt + kNearBox - 1) / kNearBox; }
     __host__ __device__ int bins() const { return (n_tgt + kNearBin - 1) / kNearBin; }
 };
 
 bool near_cheb_try(int mode, int precision, int n_src, int n_tgt);
 size_t near_cheb_bytes(int mode, int n_src, int n_tgt);
-// u, v: the scalar field's parts (scalar mode), else nullptr
-NearWs near_cheb_carve(void *base, int mode, const GridPtrs &cs, int n_src, const GridPtrs &ct, int n_tgt,
-                       const double *u, const double *v);
+NearWs near_cheb_carve(void *base, int mode, int n_src, const GridPtrs &ct, int n_tgt);
 
 }  // namespace pypo

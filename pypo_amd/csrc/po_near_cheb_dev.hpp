@@ -49,6 +49,36 @@ __device__ __forceinline__ void near_coords(const double (&e)[3][3], const doubl
     b = x[1] * f;
 }
 
+// Box of one workgroup's share of the targets, for the plan; a target that is
+// not finite leaves NaN.
+__device__ __forceinline__ void near_target_box(const NearWs &w, int block, float *scratch) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {INFINITY, INFINITY, INFINITY}, bad = 0.f;
+    const double *p[3] = {w.tx, w.ty, w.tz};
+#pragma unroll
+    for (int j = 0; j < kNearBox / TILE; j++) {
+        const int i = block * kNearBox + j * TILE + threadIdx.x;
+        if (i >= w.n_tgt) break;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const float x = (float)p[q][i];
+            lo[q] = fminf(lo[q], x);
+            hi[q] = fminf(hi[q], -x);
+            if (!(fabsf(x) < 1e30f)) bad = -1.f;
+        }
+    }
+    bad = block_min(bad, scratch);
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        lo[q] = block_min(lo[q], scratch);
+        hi[q] = -block_min(hi[q], scratch);
+    }
+    if (threadIdx.x == 0) {
+        float *o = w.box + 6 * (size_t)(w.src_tiles() + block);
+        for (int q = 0; q < 3; q++) { o[q] = lo[q]; o[3 + q] = hi[q]; }
+        if (bad < 0.f) o[0] = __builtin_nanf("");
+    }
+}
+
 // Patch of (a, b).
 __device__ __forceinline__ int near_patch(const NearPlan &pl, double a, double b, int &ip, int &jp) {
     ip = min(pl.pa - 1, max(0, (int)((a - pl.a0) / pl.da)));

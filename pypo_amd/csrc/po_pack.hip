@@ -6,7 +6,8 @@
 // weight of Propagation.h:1123-1135 (half on xu edges; half on yv edges
 // unless the grid is uv) and A the area element.  A second pass writes one
 // TileMeta per 256 records (normal cone, any non-zero M), and where a
-// Chebyshev grid is tried the boxes of their positions and of the targets.  HBM-bound:
+// Chebyshev grid is tried the boxes of their positions and of the targets (with
+// the records for scalar ones).  HBM-bound:
 // 152 B read and 96 B (FP32 records) or 144 B (FP64) written per source.
 //
 // Records go out in serpentine order (grid rows alternately reversed): the
@@ -15,6 +16,7 @@
 // follower phase needs for groups of four that span a row end.
 
 #include "po_cheb_dev.hpp"
+#include "po_near_cheb_dev.hpp"
 
 namespace pypo {
 namespace {
@@ -58,26 +60,44 @@ __global__ __launch_bounds__(256) void k_pack64(GridPtrs cs, int n, Bundle12 cur
 
 __global__ __launch_bounds__(256) void k_pack_s32(GridPtrs cs, int n, const double *__restrict__ ur,
                                                   const double *__restrict__ ui, int gmode, int ncx,
-                                                  int ncy, SrcRecS32 *__restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+                                                  int ncy, SrcRecS32 *__restrict__ out, NearWs w) {
+    __shared__ float scratch[4];
+    if ((int)blockIdx.x >= n_tiles(n)) {   // behind the records: boxes of the targets
+        near_target_box(w, blockIdx.x - n_tiles(n), scratch);
+        return;
+    }
+    const int at = blockIdx.x * blockDim.x + threadIdx.x, i = min(at, n - 1);
     double wa = trapezoid_weight(i, gmode, ncx, ncy) * cs.area[i];
     SrcRecS32 r;
     r.x = cs.x[i]; r.y = cs.y[i]; r.z = cs.z[i];
     r.ur = (float)(wa * ur[i]); r.ui = (float)(wa * ui[i]);
-    out[packed_slot(i, n, ncx, ncy)] = r;
+    if (at < n) out[packed_slot(i, n, ncx, ncy)] = r;
+    if (w.plan) {
+        // an infinite field keeps the sums' own infinities and NaN: no box, no plan
+        const double p[3] = {fabsf(r.ur) < INFINITY && fabsf(r.ui) < INFINITY ? r.x : NAN, r.y, r.z};
+        position_box(w.box, blockIdx.x, p, at < n, scratch);
+    }
 }
 
 __global__ __launch_bounds__(256) void k_pack_s64(GridPtrs cs, int n, const double *__restrict__ ur,
                                                   const double *__restrict__ ui, int gmode, int ncx,
-                                                  int ncy, SrcRecS64 *__restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+                                                  int ncy, SrcRecS64 *__restrict__ out, NearWs w) {
+    __shared__ float scratch[4];
+    if ((int)blockIdx.x >= n_tiles(n)) {   // behind the records: boxes of the targets
+        near_target_box(w, blockIdx.x - n_tiles(n), scratch);
+        return;
+    }
+    const int at = blockIdx.x * blockDim.x + threadIdx.x, i = min(at, n - 1);
     double wa = trapezoid_weight(i, gmode, ncx, ncy) * cs.area[i];
     SrcRecS64 r;
     r.x = cs.x[i]; r.y = cs.y[i]; r.z = cs.z[i];
     r.ur = wa * ur[i]; r.ui = wa * ui[i]; r.pad = 0.0;
-    out[packed_slot(i, n, ncx, ncy)] = r;
+    if (at < n) out[packed_slot(i, n, ncx, ncy)] = r;
+    if (w.plan) {
+        // an infinite field keeps the sums' own infinities and NaN: no box, no plan
+        const double p[3] = {fabs(r.ur) < 1e300 && fabs(r.ui) < 1e300 ? r.x : NAN, r.y, r.z};
+        position_box(w.box, blockIdx.x, p, at < n, scratch);
+    }
 }
 
 template <class Rec>
@@ -113,10 +133,11 @@ __device__ __forceinline__ void rec_normal_m<SrcRec64>(const SrcRec64 &r, float 
 // One workgroup per tile of 256 records.
 template <class Rec>
 __global__ __launch_bounds__(256) void k_tile_meta(const Rec *__restrict__ recs, int n,
-                                                   TileMeta *__restrict__ meta, ChebWs w) {
+                                                   TileMeta *__restrict__ meta, ChebWs w, NearWs nw) {
     __shared__ float scratch[4];
     if ((int)blockIdx.x >= n_tiles(n)) {   // behind the tiles: boxes of the targets
-        target_box(w, blockIdx.x - n_tiles(n), scratch);
+        if (nw.plan) near_target_box(nw, blockIdx.x - n_tiles(n), scratch);
+        else target_box(w, blockIdx.x - n_tiles(n), scratch);
         return;
     }
     const int i = blockIdx.x * TILE + threadIdx.x;
@@ -137,10 +158,11 @@ __global__ __launch_bounds__(256) void k_tile_meta(const Rec *__restrict__ recs,
         t.pad1 = 0;
         meta[blockIdx.x] = t;
     }
-    if (w.plan) {
+    float *box = nw.plan ? nw.box : w.src_box;
+    if (box) {
         double p[3] = {0.0, 0.0, 0.0};
         if (valid) { p[0] = recs[i].x; p[1] = recs[i].y; p[2] = recs[i].z; }
-        position_box(w, blockIdx.x, p, valid, scratch);
+        position_box(box, blockIdx.x, p, valid, scratch);
     }
 }
 
@@ -156,12 +178,13 @@ size_t packed_bytes(int mode, int precision, int n_src) {
 }
 
 int launch_pack_sources(int precision, const GridPtrs &cs, int n_src, const Bundle12 &cur,
-                        int gmode, int ncx, int ncy, void *packed, hipStream_t st, const ChebWs *cheb) {
+                        int gmode, int ncx, int ncy, void *packed, hipStream_t st, const ChebWs *cheb, const NearWs *near) {
     PYPO_REQUIRE(n_src > 0 && (long long)ncx * ncy == n_src, ERR_ARG,
                  "source n_cells do not match the source size");
     int blocks = (n_src + 255) / 256;
     const ChebWs w = cheb ? *cheb : ChebWs{};
-    const int meta_blocks = n_tiles(n_src) + (w.plan ? w.boxes() : 0);
+    const NearWs nw = near ? *near : NearWs{};
+    const int meta_blocks = n_tiles(n_src) + (nw.plan ? nw.tgt_blocks() : w.plan ? w.boxes() : 0);
     TileMeta *meta = (TileMeta *)((char *)packed +
                                   meta_offset(record_bytes(PYPO_MODE_FF, precision), n_src));
     if (precision == PYPO_PREC_FP64) {
@@ -169,13 +192,13 @@ int launch_pack_sources(int precision, const GridPtrs &cs, int n_src, const Bund
                            (SrcRec64 *)packed);
         PYPO_CHECK_LAUNCH();
         hipLaunchKernelGGL(k_tile_meta<SrcRec64>, dim3(meta_blocks), dim3(TILE), 0, st,
-                           (const SrcRec64 *)packed, n_src, meta, w);
+                           (const SrcRec64 *)packed, n_src, meta, w, nw);
     } else {
         hipLaunchKernelGGL(k_pack32, dim3(blocks), dim3(256), 0, st, cs, n_src, cur, gmode, ncx, ncy,
                            (SrcRec32 *)packed);
         PYPO_CHECK_LAUNCH();
         hipLaunchKernelGGL(k_tile_meta<SrcRec32>, dim3(meta_blocks), dim3(TILE), 0, st,
-                           (const SrcRec32 *)packed, n_src, meta, w);
+                           (const SrcRec32 *)packed, n_src, meta, w, nw);
     }
     PYPO_CHECK_LAUNCH();
     return 0;
@@ -183,16 +206,17 @@ int launch_pack_sources(int precision, const GridPtrs &cs, int n_src, const Bund
 
 int launch_pack_scalar(int precision, const GridPtrs &cs, int n_src, const double *ur,
                        const double *ui, int gmode, int ncx, int ncy, void *packed,
-                       hipStream_t st) {
+                       hipStream_t st, const NearWs *near) {
     PYPO_REQUIRE(n_src > 0 && (long long)ncx * ncy == n_src, ERR_ARG,
                  "source n_cells do not match the source size");
-    int blocks = (n_src + 255) / 256;
+    const NearWs w = near ? *near : NearWs{};
+    const int blocks = n_tiles(n_src) + (w.plan ? w.tgt_blocks() : 0);
     if (precision == PYPO_PREC_FP64)
         hipLaunchKernelGGL(k_pack_s64, dim3(blocks), dim3(256), 0, st, cs, n_src, ur, ui, gmode, ncx,
-                           ncy, (SrcRecS64 *)packed);
+                           ncy, (SrcRecS64 *)packed, w);
     else
         hipLaunchKernelGGL(k_pack_s32, dim3(blocks), dim3(256), 0, st, cs, n_src, ur, ui, gmode, ncx,
-                           ncy, (SrcRecS32 *)packed);
+                           ncy, (SrcRecS32 *)packed, w);
     PYPO_CHECK_LAUNCH();
     return 0;
 }
