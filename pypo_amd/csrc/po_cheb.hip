@@ -158,11 +158,19 @@ __global__ __launch_bounds__(1024) void k_cheb_plan(PlanIn in, ChebWs w) {
         if (lane == 0) atomicMin(&row, first);
     }
     __syncthreads();
+    // ... and 256 targets scattered over all of them (one wave a SIMD: sixteen waves'
+    // sines took 6 us): the rule below counts on rows, and first targets in a row
+    // say little of the others (a scan back and forth).
+    bool rows = row >= 16 && row <= kChebMaxRow && in.n_tgt % row == 0 && pl.na * row <= min(kChebMaxRows, in.n_tgt);
+    if (rows && tid < 256) {
+        const double g = tid * 0.6180339887498949;
+        rows = cheb_in_row(w, min(in.n_tgt - 1, (int)((g - floor(g)) * in.n_tgt)), row, tol);
+    }
+    rows = __syncthreads_and(rows);
     if (tid == 0) {
         pl.has_m = flags[1];
         pl.row_tol = tol;
-        pl.row = row >= 16 && row <= kChebMaxRow && in.n_tgt % row == 0 &&
-                         pl.na * row <= min(kChebMaxRows, in.n_tgt) ? row : 0;
+        pl.row = rows ? row : 0;
         const double terms = pl.row ? pl.na : pl.n;
         const int tiles = ((pl.na + kMomA - 1) / kMomA) * ((pl.nb + kMomB - 1) / kMomB);
         const double eval = in.moments > 0.0 ? (tiles + kMomTiles - 1) / kMomTiles * in.moments * 64.0

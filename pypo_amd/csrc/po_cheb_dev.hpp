@@ -110,21 +110,25 @@ __device__ __forceinline__ void cheb_reduce(const ChebWs &w, const double *__res
     }
 }
 
-// Checks the rows a plan supposes (pl.row): each target's a against its row's
+// Whether target t stands where rows of `row` put it: its a against its row's
 // first target and its b against the first row's, within the rounding of theta
 // and phi.
+__device__ __forceinline__ bool cheb_in_row(const ChebWs &w, int t, int row, double tol) {
+    const int i = t / row, j = t - i * row;
+    double a, b, a0, b0, x;
+    target_ab(w.tgt_th, w.tgt_ph, t, a, b);
+    target_ab(w.tgt_th, w.tgt_ph, i * row, a0, x);
+    target_ab(w.tgt_th, w.tgt_ph, j, x, b0);
+    return fabs(a - a0) <= tol && fabs(b - b0) <= tol;
+}
+
+// Checks the rows a plan supposes (pl.row) at every target.
 __device__ __forceinline__ void cheb_check_rows(const ChebWs &w, int block, int blocks) {
     const ChebPlan &pl = *w.plan;
     if (!pl.row) return;
     bool bad = false;
-    for (int t = block * TILE + threadIdx.x; t < w.n_tgt; t += blocks * TILE) {
-        const int i = t / pl.row, j = t - i * pl.row;
-        double a, b, a0, b0, x;
-        target_ab(w.tgt_th, w.tgt_ph, t, a, b);
-        target_ab(w.tgt_th, w.tgt_ph, i * pl.row, a0, x);
-        target_ab(w.tgt_th, w.tgt_ph, j, x, b0);
-        bad |= !(fabs(a - a0) <= pl.row_tol && fabs(b - b0) <= pl.row_tol);
-    }
+    for (int t = block * TILE + threadIdx.x; t < w.n_tgt; t += blocks * TILE)
+        bad |= !cheb_in_row(w, t, pl.row, pl.row_tol);
     if (bad) *w.not_rows = 1;
 }
 

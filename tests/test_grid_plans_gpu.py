@@ -239,3 +239,24 @@ def test_gradient_plan_counts_the_moments(grids, n_dish, n_ff, ff_deg, far):
     E = torch.randn((12, n_ff * n_ff), dtype=torch.float64, device="cuda", generator=gen)
     prob.power_grad(torch.zeros(n_dish * n_dish, dtype=torch.float64, device="cuda"), E, E[0])
     assert grids()[0] == far
+
+
+def test_far_plan_of_a_scan_back_and_forth(grids):
+    """Few sources, many targets: the series pays along rows of equal azimuth
+    only.  Rows alternately reversed are none, though the first targets look like
+    one: the sums at the targets then, and the same field."""
+    import torch
+    from pypo_amd import device as D
+    src, ff = _plane(16.0, 36), _aoe([-12.0, 12.0], [-12.0, 12.0], 701, 703)
+    g_s, g_t = D.generate_grid(src), D.generate_grid(ff)
+    c = D.currents_tensor(_aperture(36, 1.0))
+    ref = D.propagate("FF", g_s, g_t, c, src, K)
+    info = grids()
+    assert info[0] == ON and info[3] == 703
+    order = torch.arange(701 * 703, device="cuda").view(701, 703).clone()
+    order[1::2] = order[1::2].flip(1)
+    order = order.reshape(-1)
+    out = D.propagate("FF", g_s, g_t[:, order].contiguous(), c, src, K)
+    print(info, grids())
+    assert grids()[0] == OFF
+    assert ((out - ref[:, order]).abs().max() / ref.abs().max()).item() <= TOL["mixed"]
