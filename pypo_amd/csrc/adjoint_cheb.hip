@@ -326,7 +326,9 @@ int launch_adj_near(int precision, const NearWs &near, const void *feed64, int n
     NearWs w = near;
     w.nodes_only = true;
     const TileMeta *meta = (const TileMeta *)((const char *)feed64 + meta_offset(sizeof(SrcRec64), n_feed));
-    const SumPlan p{1, std::min((n_dish + TILE - 1) / TILE, kNearMaxNodes / TILE), n_tiles(n_feed), TILE};
+    // what the sums may launch; splits are grid.y, 65 536 at most, and a thousand
+    // already fill the chip for one block of nodes
+    const SumPlan p{1, std::min((n_dish + TILE - 1) / TILE, kNearMaxNodes / TILE), std::min(n_tiles(n_feed), 1024), TILE};
     const double carrier = tdir * k / kTwoPi;
     int err;
     if ((err = launch_near_cheb_plan(PYPO_MODE_JM, precision, PYPO_PREC_FP64, p, meta, n_feed, k, partial_bytes,
