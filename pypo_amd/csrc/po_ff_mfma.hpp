@@ -22,9 +22,8 @@
 // scaled per 256-source tile by a power of two that takes the tile's largest
 // component (TileMeta::cmax) to [2^13, 2^14): FP16's spacing stays at 2^-24
 // below 2^-14, so lo would round every component, however small, to 2^-25 of
-// the largest if that were taken to 1, and only to 2^-39 like this.  The FP32 tile
-// sums are multiplied back and folded into FP64 after every tile, like the
-// vector kernel's.  The operand split costs three VALU instructions per pair
+// the largest if that were taken to 1, and only to 2^-39 like this.  The FP32
+// sums are multiplied back and folded into FP64 twice a tile.  The operand split costs three VALU instructions per pair
 // against the twelve FP32 FMAs the vector kernel spends on the products.
 //
 // Phase.  The four sources a lane takes per K-step are consecutive records,
@@ -69,6 +68,12 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int KSTEPS = TILE / 16;   // 16 sources (32 K rows: cos and sin) per MFMA
+
+// K-steps whose FP32 sums are folded into FP64 at once.  Half a tile: at a few
+// Chebyshev nodes that hold the main beam the rounding of a whole tile's
+// partial sum does not average out over targets, and a gradient through the
+// difference of two such powers was off by 2.7e-7 instead of 2.2e-7.
+constexpr int FOLD_KSTEPS = KSTEPS / 2;
 
 // Largest bound on the follower phase sums (revolutions): FP32 rounds such a
 // sum to 2^-24 * 8 = 5e-7 revolutions at worst.
@@ -218,16 +223,16 @@ __device__ __forceinline__ void ff_kstep(const TileXYZ &tx, const half8 &b_hi, c
     }
 }
 
-// The first ksteps K-steps (16 sources each) of a tile, all in the follower form or none (one
+// K-steps k0 to k1 (16 sources each) of a tile, all in the follower form or none (one
 // loop body per form keeps the accumulators in place).
 template <int MB, bool MASK, bool FAST>
 __device__ __forceinline__ void ff_tile_mfma(const TileXYZ &tx, const half8 (*bhi)[64], const half8 (*blo)[64],
                                              int lane, const double (&qx)[MB], const double (&qy)[MB],
                                              const double (&qz)[MB], const float4 *tq, int lt0,
-                                             floatx4 (&acc)[MB], int ksteps) {
+                                             floatx4 (&acc)[MB], int k0, int k1) {
     const int kb = lane >> 4;
 #pragma unroll 1
-    for (int ks = 0; ks < ksteps; ks++) {
+    for (int ks = k0; ks < k1; ks++) {
         const int slot = b_slot(ks, lane);
         const half8 b_hi = bhi[ks][slot], b_lo = blo[ks][slot];
         ff_kstep<MB, MASK, FAST>(tx, b_hi, b_lo, ks * 16 + kb * 4, qx, qy, qz, tq, lt0, acc);
@@ -299,11 +304,17 @@ __device__ __forceinline__ void ff_mfma_body(const SrcRec32 *__restrict__ src, c
     }
 
     const uint4 *g = reinterpret_cast<const uint4 *>(src);
+    // The next tile's records are fetched during a tile, but not with 8 M-blocks:
+    // the 24 registers they wait in were spilled ones (ff of 1 002 001 sources at
+    // 59 x 59 nodes 1681 us with, 1638 without; 1686 with the second fold), and
+    // eight waves a CU hide the load.
+    constexpr bool PREFETCH = MB != 8;
     TileLoader<6> ld;
-    ld.load(g, s_begin + tid, s_end);
+    if (PREFETCH) ld.load(g, s_begin + tid, s_end);
     for (int base = s_begin; base < s_end; base += TILE) {
         const TileMeta tm = meta[base / TILE];
         const float inv = tile_inv_scale(tm.cmax);
+        if (!PREFETCH) ld.load(g, base + tid, s_end);
         {
             const SrcRec32 r = __builtin_bit_cast(SrcRec32, ld.buf);   // this lane's record
             // offset from the group's leader (same wave), in revolutions
@@ -330,23 +341,28 @@ __device__ __forceinline__ void ff_mfma_body(const SrcRec32 *__restrict__ src, c
             build_b(r, tid, inv, bhi, blo);
             __syncthreads();
         }
-        if (base + TILE < s_end) ld.load(g, base + TILE + tid, s_end);
+        if (PREFETCH && base + TILE < s_end) ld.load(g, base + TILE + tid, s_end);
         const bool fast = __builtin_amdgcn_readfirstlane(tx.fast[0] & tx.fast[1] & tx.fast[2] & tx.fast[3]);
         const int lt0 = wave * 16 * MB + row;
         const int ksteps = (min(TILE, s_end - base) + 15) / 16;
-        if (cones_may_shadow(tm.ax, tm.ay, tm.az, tm.cos_half, cone)) {
-            if (fast) ff_tile_mfma<MB, true, true>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, ksteps);
-            else ff_tile_mfma<MB, true, false>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, ksteps);
-        } else {
-            if (fast) ff_tile_mfma<MB, false, true>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, ksteps);
-            else ff_tile_mfma<MB, false, false>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, ksteps);
-        }
+        const bool mask = cones_may_shadow(tm.ax, tm.ay, tm.az, tm.cos_half, cone);
         const double scale = 1.0 / (double)inv;   // a power of two: exact
+#pragma unroll 1
+        for (int k0 = 0; k0 < ksteps; k0 += FOLD_KSTEPS) {
+            const int k1 = min(ksteps, k0 + FOLD_KSTEPS);
+            if (mask) {
+                if (fast) ff_tile_mfma<MB, true, true>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, k0, k1);
+                else ff_tile_mfma<MB, true, false>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, k0, k1);
+            } else {
+                if (fast) ff_tile_mfma<MB, false, true>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, k0, k1);
+                else ff_tile_mfma<MB, false, false>(tx, bhi, blo, lane, qx, qy, qz, tq, lt0, acc, k0, k1);
+            }
 #pragma unroll
-        for (int m = 0; m < MB; m++) {
+            for (int m = 0; m < MB; m++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) tot[m][i] = __builtin_fma((double)acc[m][i], scale, tot[m][i]);
-            acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < 4; i++) tot[m][i] = __builtin_fma((double)acc[m][i], scale, tot[m][i]);
+                acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
         }
     }
     // D layout: this lane holds column `row` of targets t0 + 16 m + 4 kb + i
