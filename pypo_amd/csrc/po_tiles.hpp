@@ -10,14 +10,15 @@ namespace pypo {
 
 // Far field: six (or three, J only) complex multiply-adds of w*A*currents
 // with exp(-j t k r'.r) per pair; MASK applies the shadow test n.r >= 0
-// (Propagation.h:1719).  rx/ry/rz = r * (-t k / 2 pi) in FP64, fx/fy/fz = r.
-template <int TPL, bool HAS_M, bool MASK>
+// (Propagation.h:1719).  rx/ry/rz = r * (-t k / 2 pi) in FP64, fx/fy/fz = r.  N:
+// records of `tile` to sum.
+template <int TPL, bool HAS_M, bool MASK, int N = TILE>
 __device__ __forceinline__ void ff_tile_mixed(const SrcRec32 *tile, const double (&rx)[TPL],
                                               const double (&ry)[TPL], const double (&rz)[TPL],
                                               const float (&fx)[TPL], const float (&fy)[TPL],
                                               const float (&fz)[TPL], float (&acc)[TPL][12]) {
 #pragma unroll 2
-    for (int s = 0; s < TILE; s++) {
+    for (int s = 0; s < N; s++) {
         const SrcRec32 &r = tile[s];
         const double x = r.x, y = r.y, z = r.z;
         float cj[6], cm[6];
