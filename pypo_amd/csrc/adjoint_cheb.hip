@@ -16,12 +16,12 @@
 // patches around the feed (po_near_cheb.hpp): one H-only sum at the nodes in
 // place of the sum of H and dH at every dish point.  Errors of the node sums
 // come back smooth over a patch and do not average out over the dish, so they
-// are FP64 sums in mixed precision too (160 us, 95 us mixed).
+// are FP64 sums in mixed precision too (158 us).
 //
 // Measured on MI355X, 401^2 dish, 151^2 far field, 33^2 feed, mixed: reverse
-// sums 1926 -> 800 us (590 of them the sums at the nodes, 165 the moments),
-// currents 1356 -> 520 us (220 the series).  Gradient error against FP64 over
-// six problems of 327^2 to 426^2 dishes: rms 2.4e-7 -> 2.6e-7 of its norm.
+// sums 1926 -> 740 us (503 of them the sums at the nodes, 157 the moments),
+// currents 1356 -> 490 us (209 the series).  Gradient error against FP64 over
+// fourteen problems of 327^2 to 426^2 dishes: rms 2.2e-7 -> 2.1e-7 of its norm.
 
 #include "adjoint.hpp"
 #include "po_cheb_dev.hpp"

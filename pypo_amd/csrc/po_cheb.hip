@@ -281,8 +281,9 @@ int launch_cheb_plan(int precision, const SumPlan &p, const TileMeta *meta, int 
     in.max_items = (int)std::min((long long)p.tblocks * p.splits, (1LL << 30));
     in.max_partials = (long long)(partial_bytes / sizeof(double));
     in.kabs = std::fabs(rev_scale) * kTwoPi;
-    in.q = f64 ? 8.9 : 6.9;
-    in.p = f64 ? 10.05 : 3.05;
+    const NodeRule &rule = f64 ? kNodesFp64 : kNodesMixed;
+    in.q = rule.q;
+    in.p = rule.p;
     in.cycles = cost.cycles;
     in.fixed = cost.fixed_us * 64.0 * kSimdHz * 1e-6 / cost.cycles;
     in.extra = cost.extra;

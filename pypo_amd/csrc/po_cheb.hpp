@@ -15,14 +15,15 @@
 //
 // Node count.  The interpolant of exp(j K x) at n Chebyshev nodes of [-1, 1]
 // is off by at most 4 sum_{i >= n} |J_i(K)|; n = ceil(K + q K^(1/3) + p) keeps
-// that below eps = 1e-10 for q, p = 7.7, 3.5 (mixed precision, whose FP32 sums
-// are good to 1e-7) and below 3e-15 for 8.9, 10.05 (FP64), for all K up to 160.
+// that below 1.6e-9 for kNodesMixed (mixed precision, whose FP32 sums are good
+// to 1e-7) and below 1.5e-15 for kNodesFp64, for all K up to 160.
 // The phase is not linear in a and b; what matters is its growth over the
 // Bernstein ellipse of that convergence, imaginary extent eta = sqrt(n^2 -
 // K^2) / (K / h), where |dr_x/da| <= cosh eta, |dr_y/da| <= |a b| / 3 cosh eta
 // and |dr_z/da| <= (|a| + eta) cosh eta.  The plan iterates K with those
 // bounds.  Over 250 random boxes (to 1.5 rad off axis) and source extents (to
-// 1e4 rad), the worst error was a sixth of eps.
+// 1e4 rad), the worst error was 5.9e-11 mixed, 5.7e-12 FP64 (which phases of 1e4
+// rad round to).
 //
 // When it is taken.  The decision needs the extents of the sources and of the
 // directions, which live on the device, so it is made there: the pack
@@ -32,7 +33,9 @@
 // targets as they come, when
 //   * some tile of sources could be shadowed in part of the box (n.r of either
 //     sign): the shadow test makes the sums discontinuous in r;
-//   * an extent or a current is not finite, or the box reaches beyond 1.5 rad;
+//   * an extent is not finite, a current infinite (one that is not a number
+//     spoils every node, and so every target it would), or the box reaches beyond
+//     1.5 rad;
 //   * the nodes would cost more than the targets they stand for (the rule is at
 //     cheb_pays).
 //
@@ -41,9 +44,10 @@
 // against it, and the series is then summed along b once per column.
 //
 // Measured on MI355X: 1 002 001 sources -> 251 001 targets over +-10.5 beam
-// widths, 59 x 59 nodes, 91.6 -> 1.71 ms mixed (error against 64 bits 9.5e-8
-// both ways), of which the node sums 1.6 ms; 90 300 -> 40 401 in FP64 5.14 ->
-// 0.72 ms; 89 999 -> 31 313 with J and M over +-15 beam widths 1.27 -> 0.39 ms.
+// widths, 59 x 59 nodes, 91.6 -> 1.69 ms mixed (error against 64 bits 9.5e-8 ->
+// 7.2e-8), of which the node sums 1.5 ms; 90 300 -> 40 401 in FP64 5.14 ->
+// 0.72 ms; 89 999 -> 31 313 with J and M over +-15 beam widths 1.27 -> 0.385 ms.
+// Where the plan stays off it costs some 15 us.
 // The row form: the two-dimensional series took 540, 260 and 270 us of these,
 // the rows 37, 31 and 44 us.
 #pragma once
@@ -51,6 +55,10 @@
 #include "common.hpp"
 
 namespace pypo {
+
+// Node counts of the far and the near grids: q and p of the rule, and ln(4 / eps).
+struct NodeRule { double q, p, log_eps; };
+constexpr NodeRule kNodesMixed{6.9, 3.05, 21.1}, kNodesFp64{8.9, 10.05, 34.8};
 
 constexpr int kChebMaxNodes = 32768;    // na nb, also the workspace's size
 constexpr int kChebMaxAxis = 224;       // na, nb

@@ -764,9 +764,10 @@ int launch_near_cheb_plan(int mode, int precision, int sums, const SumPlan &p, c
     in.rows = near_rows(mode);
     in.max_partials = (long long)(partial_bytes / sizeof(double)) / (mode == PYPO_MODE_SCALAR ? 1 : 12 / in.rows);
     in.kabs = (float)kabs;
-    in.q = f64 ? 8.9f : 6.9f;
-    in.p = f64 ? 10.05f : 3.05f;
-    in.log_eps = f64 ? 34.8f : 21.1f;           // ln(4 / 3e-15), ln(4 / 3e-9)
+    const NodeRule &rule = f64 ? kNodesFp64 : kNodesMixed;
+    in.q = (float)rule.q;
+    in.p = (float)rule.p;
+    in.log_eps = (float)rule.log_eps;
     for (int n = 1; n < kNearSmall; n++) {
         // 2 (K / 2)^n / n! = eps
         in.small[n] = 2.f * std::exp((std::lgamma(n + 1.f) + 0.693f - in.log_eps) / n);

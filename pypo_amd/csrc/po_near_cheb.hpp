@@ -34,16 +34,17 @@
 // The plan is made on the device, like the far field's, and is off where
 //   * R_min < 3 rho, the targets spread more than 1.5 rad around the axis, or
 //     some pair may be in shadow;
-//   * an extent or a current is not finite;
+//   * an extent is not finite or a current infinite (one that is not a number
+//     spoils every node, and so every target it would);
 //   * nodes and series would cost more than the sums at the targets.
 //
 // Targets of 200 000 points and more are evaluated in the order of their
 // patches (a counting sort): in grid order a wave of a polar grid meets three.
 //
 // Measured on MI355X (node sums / series / whole call, before): JM 1089 ->
-// 1 002 001 mixed 133 / 250 / 530 us (2 410), error against 64 bits 4.2e-7
-// (4.9e-7); EHP 10 201 -> 640 800 566 / 386 / 986 us (20 150), 3.1e-8
-// (3.2e-8); scalar 10 201 -> 160 801 151 / 157 / 368 us (1 253), 2.0e-7
+// 1 002 001 mixed 122 / 187 / 472 us (2 410), error against 64 bits 1.3e-7
+// (4.8e-7); EHP 10 201 -> 640 800 491 / 322 / 950 us (20 150), 2.3e-8
+// (3.2e-8); scalar 10 201 -> 160 801 133 / 93 / 304 us (1 253), 2.0e-7
 // (2.2e-7).
 #pragma once
 
