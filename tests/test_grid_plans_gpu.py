@@ -1,5 +1,5 @@
 """Which calls the Chebyshev grids take (pypo_hip_last_grids), against the CPU
-checker on both sides of the decision, at sizes well inside the range where a
+oracle on both sides of the decision, at sizes well inside the range where a
 plan is tried.
 
 Tolerances.  Mixed: FP32 phases (2e-7 rad), sines and products of terms whose
@@ -78,7 +78,7 @@ NEAR = {
 }
 
 
-def _checker(port, mode, g_s, cells, vals, pts):
+def _oracle(port, mode, g_s, cells, vals, pts):
     if mode != "scalar":
         return OB.propagate_on_grids(port, mode, g_s, cells, pts, vals, K)
     _, nu, nv = cells                       # Propagation.h:1279-1331
@@ -110,7 +110,7 @@ def test_near_plans(grids, port, name, mode, prec, state):
     n_t = g_t.shape[1]
     idx = np.unique(np.concatenate([np.random.default_rng(1).integers(0, n_t, 150), [0, n_t - 1]]))
     pts = g_t[:, torch.as_tensor(idx, device="cuda")].cpu().numpy()
-    ref = _checker(port, mode, g_s.cpu().numpy(), (int(src["gmode"]), n, n), vals.cpu().numpy(), pts)
+    ref = _oracle(port, mode, g_s.cpu().numpy(), (int(src["gmode"]), n, n), vals.cpu().numpy(), pts)
     step = 2 if mode == "scalar" else (3 if mode == "EHP" else 6)
     worst = 0.0
     for g in range(0, ref.shape[0], step):

@@ -1,5 +1,5 @@
 """Near fields of sources much smaller than a wavelength, on targets within and
-around the near zone, against the CPU checker: there the 1 / (k R) and
+around the near zone, against the CPU oracle: there the 1 / (k R) and
 1 / (k R)^2 terms set how fast the field changes with the distance, not the
 sources' extent.  Sizes at which the Chebyshev patches are tried.
 
@@ -32,7 +32,7 @@ def _plane(h, n, z):
                                             (1e-3, 0.1, 0.1), (1e-2, 0.4, 0.5), (0.1, 1.3, 0.3)])
 @pytest.mark.parametrize("mode,prec,exp", [("JM", "mixed", "fwd"), ("EH", "mixed", "bwd"), ("JM", "fp64", "bwd"),
                                            ("JMEH", "fp64", "fwd")])
-def test_point_like_source_matches_checker(hip, port, hw, dist, spread, mode, prec, exp):
+def test_point_like_source_matches_oracle(hip, port, hw, dist, spread, mode, prec, exp):
     import torch
     from pypo_amd import device as D
     src = _plane(hw, N_S, 0.0)
